@@ -1,8 +1,10 @@
 /*
  * lbm_batch.h -- batches of many small, uneven lattice-Boltzmann domains in
- * one launch per step (one block per tile or a persistent grid, as the
- * autotuner chooses), K steps plus the convergence check captured in one
- * hipGraph (part of liblbm_hip.so).
+ * one launch for all of them, K steps plus the convergence check captured in
+ * one hipGraph (part of liblbm_hip.so).  Plain D2Q9 steps run several per
+ * launch on tiles held in LDS; the steps of a convergence check, D3Q19
+ * batches and those with faces that form has no rule for run one per launch
+ * (one block per tile or a persistent grid, as the autotuner chooses).
  *
  * No reference counterpart: SFCMM/LBM runs one domain per process
  * (src/lbm/solver.cpp:176-214).  Each domain here is a structured box with its
@@ -41,7 +43,7 @@ typedef struct {
 
 int lbm_batch_create(int32_t lattice, int32_t storage, const lbm_domain_desc *doms, int32_t ndom, lbm_batch **out);
 
-/* Autotuner: times every candidate tiling (2D tiles of 256 cells and width
+/* Autotuner of the steps taken one per launch: times every candidate tiling (2D tiles of 256 cells and width
  * 16/32/64/128/256; tile_x 1: banded, 16x16 tiles along both x faces and
  * 64x4 tiles between; tile_x 0: row runs, 256 consecutive cells of a
  * rectangle of cells of one class -- interior, boundary, next to a solid;

@@ -75,6 +75,10 @@ struct lbm_batch {
   std::vector<std::vector<uint8_t>> cclass;       // every domain's cell classes (tiles)
   std::vector<std::vector<BatchTile>> dom_tiles;  // every domain's tiles for tiling cache_tx
   int cache_tx = -1;
+  MultiTile *mtiles_d = nullptr;  // tiles of the multi-step launches (null: single steps only)
+  int nmtiles = 0;
+  Multi2dPlan mplan{};
+  int mcls = MULTI2D_WALLS;
   int *ids_d = nullptr;  // launch lists: interior tiles, boundary tiles, every tile
   int n_int = 0, n_bnd = 0;
   int tx = 64, blocks = 0;  // blocks == 0: one block per tile
@@ -288,6 +292,51 @@ static void domain_tiles(const DomainDev &D, const std::vector<uint8_t> &cc, int
   }
 }
 
+// Tiles of the multi-step launches (k_multi2d): every active domain cut into
+// equal tiles no larger than the plan's, those without a fluid cell left
+// out.  Empty where the plain steps run one per launch: D3Q19, and batches
+// with a face that kernel has no rule for (multi2d_class).
+static std::vector<MultiTile> multi_tiles(lbm_batch *b) {
+  std::vector<MultiTile> out;
+  if (b->Q != 9) return out;
+  int nx = 0, ny = 0;
+  long long cells = 0;
+  for (int d = 0; d < b->ndom; ++d) {
+    const DomainDev &D = b->doms[d];
+    if (!b->active_h.empty() && !b->active_h[d]) continue;
+    nx = std::max(nx, D.nx);
+    ny = std::max(ny, D.ny);
+    cells += (long long)D.nx * D.ny;
+  }
+  if (!cells) return out;
+  b->mcls = MULTI2D_WALLS;  // the kernel reads every domain's masks
+  for (int d = 0; d < b->ndom; ++d) {
+    const int cls = multi2d_class(b->doms[d].face, true, cells, b->esize);
+    if (cls == MULTI2D_NONE) return out;
+    b->mcls = std::max(b->mcls, cls);
+  }
+  b->mplan = multi2d_plan(nx, ny, cells, b->esize, true);
+  for (int d = 0; d < b->ndom; ++d) {
+    if (!b->active_h.empty() && !b->active_h[d]) continue;
+    const DomainDev &D = b->doms[d];
+    const std::vector<uint8_t> &cc = b->cclass[d];
+    const int cols = (D.nx + b->mplan.tw - 1) / b->mplan.tw, rows = (D.ny + b->mplan.th - 1) / b->mplan.th;
+    // widths in whole groups of 16 cells, so that rows start on the same
+    // part of a line
+    const int w = std::min(b->mplan.tw, ((D.nx + cols - 1) / cols + 15) / 16 * 16), h = (D.ny + rows - 1) / rows;
+    for (int y0 = 0; y0 < D.ny; y0 += h)
+      for (int x0 = 0; x0 < D.nx; x0 += w) {
+        const MultiTile t{d, x0, y0, std::min(w, D.nx - x0), std::min(h, D.ny - y0)};
+        bool fluid = false;
+        for (int y = 0; y < t.h && !fluid; ++y)
+          for (int x = 0; x < t.w && !fluid; ++x) fluid = cc[(size_t)(x0 + x) + (size_t)D.nx * (y0 + y)] != CELL_SOLID;
+        if (fluid) out.push_back(t);
+      }
+  }
+  b->mplan.wide = b->mplan.wide && out.size() <= 256;  // one block per CU
+  return out;
+}
+
 // Tiles of every still-active domain (each domain's list is built once per
 // tiling and kept).  The new buffers are allocated and filled before the
 // old ones are freed, so a failed rebuild leaves the previous tiling in
@@ -322,31 +371,40 @@ static int batch_build_tiles(lbm_batch *b, int tx) {
     ids_bnd.push_back(0);
     tiles.push_back(BatchTile{0, 0, 1, 0, 0, 0, 0, 1});  // no lane active
   }
+  std::vector<MultiTile> mtiles = multi_tiles(b);
   // launch lists: the interior tiles, the boundary tiles, then every tile in
   // list order (the single-launch form)
   std::vector<int> ids(ids_int);
   ids.insert(ids.end(), ids_bnd.begin(), ids_bnd.end());
   for (int t = 0; t < (int)tiles.size(); ++t) ids.push_back(t);
   BatchTile *tiles_d = nullptr;
+  MultiTile *mtiles_d = nullptr;
   int *ids_d = nullptr;
   double *partials = nullptr;
   auto release = [&](int code, const std::string &msg) {
     if (tiles_d) (void)hipFree(tiles_d);
+    if (mtiles_d) (void)hipFree(mtiles_d);
     if (ids_d) (void)hipFree(ids_d);
     if (partials) (void)hipFree(partials);
     return bfail(b, code, msg);
   };
   if (hipMalloc(&tiles_d, tiles.size() * sizeof(BatchTile)) != hipSuccess ||
       hipMalloc(&ids_d, ids.size() * sizeof(int)) != hipSuccess ||
-      hipMalloc(&partials, tiles.size() * NSUM * sizeof(double)) != hipSuccess)
+      hipMalloc(&partials, tiles.size() * NSUM * sizeof(double)) != hipSuccess ||
+      (!mtiles.empty() && hipMalloc(&mtiles_d, mtiles.size() * sizeof(MultiTile)) != hipSuccess))
     return release(LBM_ENOMEM, "batch tiling: device allocation failed");
   if (hipMemcpy(tiles_d, tiles.data(), tiles.size() * sizeof(BatchTile), hipMemcpyHostToDevice) != hipSuccess ||
+      (!mtiles.empty() && hipMemcpy(mtiles_d, mtiles.data(), mtiles.size() * sizeof(MultiTile),
+                                    hipMemcpyHostToDevice) != hipSuccess) ||
       hipMemcpy(ids_d, ids.data(), ids.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(b->doms_d, doms.data(), doms.size() * sizeof(DomainDev), hipMemcpyHostToDevice) != hipSuccess)
     return release(LBM_EHIP, "batch tiling: upload failed");
   if (b->tiles_d) (void)hipFree(b->tiles_d);
   if (b->ids_d) (void)hipFree(b->ids_d);
   if (b->partials) (void)hipFree(b->partials);
+  if (b->mtiles_d) (void)hipFree(b->mtiles_d);
+  b->mtiles_d = mtiles_d;
+  b->nmtiles = (int)mtiles.size();
   b->tiles_d = tiles_d;
   b->ids_d = ids_d;
   b->partials = partials;
@@ -671,14 +729,40 @@ int lbm_batch_init_fields(lbm_batch *b, const double *rho, const double *u) {
   return LBM_OK;
 }
 
+// `steps` plain steps from the buffer `parity`; returns the parity the next
+// launch reads, the same as after that many single steps (every launch swaps
+// the buffers, and a graph's replays have to start where it was captured).
+static int batch_plain(lbm_batch *b, int parity, int steps) {
+  if (!b->mtiles_d) {
+    for (int s = 0; s < steps; ++s) batch_launch(b, (parity + s) & 1, 0);
+    return (parity + steps) & 1;
+  }
+  int n = (steps + b->mplan.steps - 1) / b->mplan.steps;
+  n += (n ^ steps) & 1;  // the parity that single steps end with
+  for (int i = 0; i < n; ++i) {
+    Multi2dArgs a;
+    memset(&a, 0, sizeof(a));
+    a.src = b->buf[parity];
+    a.dst = b->buf[parity ^ 1];
+    a.steps = steps / n + (i < steps % n ? 1 : 0);
+    a.ntiles = b->nmtiles;
+    a.tiles = b->mtiles_d;
+    a.doms = b->doms_d;
+    a.active = b->active_d;
+    a.links = b->links;
+    dispatch_s<Multi2dL>(b->storage, a, b->stream, b->mcls, b->mplan.wide);
+    parity ^= 1;
+  }
+  return parity;
+}
+
 static int batch_capture(lbm_batch *b, int interval, double tol) {
   batch_drop_graph(b);
   hipGraph_t g;
   BHIPCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeGlobal));
-  for (int s = 0; s < interval; ++s) {
-    const int mode = s == interval - 2 ? 1 : (s == interval - 1 ? 2 : 0);
-    batch_launch(b, (b->cur + s) & 1, mode);
-  }
+  const int parity = batch_plain(b, b->cur, interval - 2);
+  batch_launch(b, parity, 1);
+  batch_launch(b, parity ^ 1, 2);
   hipLaunchKernelGGL(k_domain_finalize, dim3((b->ndom + 255) / 256), dim3(256), 0, b->stream, (const DomainDev *)b->doms_d,
                      b->ndom, (const double *)b->partials, b->ntiles, b->active_d, b->res_d, b->mass_d, b->conv_d,
                      (const long long *)b->cycle_d, tol);
@@ -807,7 +891,7 @@ int lbm_batch_destroy(lbm_batch *b) {
     if (b->buf[k]) (void)hipFree(b->buf[k]);
     if (b->snap[k]) (void)hipFree(b->snap[k]);
   }
-  void *ptrs[] = {b->flags, b->links, b->doms_d, b->tiles_d, b->ids_d, b->active_d, b->res_d, b->mass_d, b->partials, b->conv_d, b->cycle_d};
+  void *ptrs[] = {b->flags, b->links, b->doms_d, b->tiles_d, b->mtiles_d, b->ids_d, b->active_d, b->res_d, b->mass_d, b->partials, b->conv_d, b->cycle_d};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   if (b->stream) (void)hipStreamDestroy(b->stream);

@@ -103,29 +103,117 @@ struct Moments {
   C drho, rho, ux, uy, uz;
 };
 
-template <int Q, typename C, typename R>
+// c_j . (x, y, z): only the terms c_j has (a product with a zero component is
+// an instruction the compiler must keep).
+template <int Q, typename C>
+__device__ __forceinline__ C cdot(int j, C x, C y, C z) {
+  using L = Lat<Q>;
+  C s = 0;
+  if (L::cx[j]) s = L::cx[j] > 0 ? x : -x;
+  if (L::cy[j]) s = L::cx[j] ? (L::cy[j] > 0 ? s + y : s - y) : (L::cy[j] > 0 ? y : -y);
+  if (L::cz[j]) s = (L::cx[j] || L::cy[j]) ? (L::cz[j] > 0 ? s + z : s - z) : (L::cz[j] > 0 ? z : -z);
+  return s;
+}
+
+// Whether population j is the member of its pair (j, opp j) whose first
+// non-zero component is +1.
+template <int Q>
+__host__ __device__ constexpr bool leads(int j) {
+  using L = Lat<Q>;
+  return L::cx[j] ? L::cx[j] > 0 : (L::cy[j] ? L::cy[j] > 0 : L::cz[j] > 0);
+}
+
+// 1 / x in FP64: the hardware's estimate, Newton steps and the fix-up of
+// zeros and infinities.  With three steps the same instructions on the same
+// values as the compiler's quotient, without its scaling (which a density
+// never needs); two leave it within an ulp.
+template <int STEPS>
+__device__ __forceinline__ double reciprocal(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+#pragma unroll
+  for (int i = 0; i < STEPS; ++i) r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  return __builtin_amdgcn_div_fixup(r, x, 1.0);
+}
+template <int STEPS>
+__device__ __forceinline__ float reciprocal(float x) {
+  return 1.0f / x;
+}
+
+// The FP64 storage form works on the pairs: their sum and difference give
+// the density and the momentum (39 additions instead of 48 on D3Q19).  The
+// smaller storage forms keep the population order: there the last bit of the
+// arithmetic now and then decides a stored bit, and a flipped one spreads
+// until the rounding errors of two orders have nothing in common.
+// FORCE false: no body force (the F arguments are not read).
+template <int Q, typename C, bool FORCE = true, typename R>
 __device__ __forceinline__ Moments<Q, C> moments(const R (&h)[Q], C Fx, C Fy, C Fz) {
   using L = Lat<Q>;
   C drho = 0, jx = 0, jy = 0, jz = 0;
+  constexpr bool PAIRS = std::is_same<R, double>::value;
+  if constexpr (PAIRS) {
+    drho = C(h[Q - 1]);
+    bool fx = true, fy = true, fz = true;  // first term of each sum (unrolled: no additions to zero)
 #pragma unroll
-  for (int j = 0; j < Q; ++j) drho += C(h[j]);
+    for (int j = 0; j < Q - 1; ++j) {
+      if (!leads<Q>(j)) continue;
+      const C a = C(h[j]), b = C(h[L::opp[j]]), d = a - b;
+      drho += a + b;
+      if (L::cx[j]) { jx = fx ? d : jx + d; fx = false; }
+      if (L::cy[j]) { jy = fy ? (L::cy[j] > 0 ? d : -d) : (L::cy[j] > 0 ? jy + d : jy - d); fy = false; }
+      if (L::cz[j]) { jz = fz ? (L::cz[j] > 0 ? d : -d) : (L::cz[j] > 0 ? jz + d : jz - d); fz = false; }
+    }
+  } else {
 #pragma unroll
-  for (int j = 0; j < Q - 1; ++j) {
-    if (L::cx[j] == 1) jx += C(h[j]);
-    if (L::cx[j] == -1) jx -= C(h[j]);
-    if (L::cy[j] == 1) jy += C(h[j]);
-    if (L::cy[j] == -1) jy -= C(h[j]);
-    if (L::cz[j] == 1) jz += C(h[j]);
-    if (L::cz[j] == -1) jz -= C(h[j]);
+    for (int j = 0; j < Q; ++j) drho += C(h[j]);
+#pragma unroll
+    for (int j = 0; j < Q - 1; ++j) {
+      if (L::cx[j] == 1) jx += C(h[j]);
+      if (L::cx[j] == -1) jx -= C(h[j]);
+      if (L::cy[j] == 1) jy += C(h[j]);
+      if (L::cy[j] == -1) jy -= C(h[j]);
+      if (L::cz[j] == 1) jz += C(h[j]);
+      if (L::cz[j] == -1) jz -= C(h[j]);
+    }
   }
   Moments<Q, C> m;
   m.drho = drho;
   m.rho = C(1) + drho;
-  const C inv = C(1) / m.rho;
-  m.ux = (jx + C(0.5) * Fx) * inv;
-  m.uy = (jy + C(0.5) * Fy) * inv;
-  m.uz = (jz + C(0.5) * Fz) * inv;
+  const C inv = reciprocal<PAIRS ? 2 : 3>(m.rho);
+  if (FORCE) {
+    m.ux = (jx + C(0.5) * Fx) * inv;
+    m.uy = (jy + C(0.5) * Fy) * inv;
+    m.uz = (jz + C(0.5) * Fz) * inv;
+  } else {
+    m.ux = jx * inv;
+    m.uy = jy * inv;
+    m.uz = L::D == 3 ? jz * inv : C(0);
+  }
   return m;
+}
+
+// The relaxation's factors: 1 - omega and omega times the weights of the
+// axis, the diagonal and the rest populations.
+template <int Q, typename C>
+struct Relax {
+  C omega, keep, axis, diag, rest;
+};
+template <int Q, typename C>
+__device__ __forceinline__ Relax<Q, C> relax(C omega) {
+  using L = Lat<Q>;
+  return Relax<Q, C>{omega, C(1) - omega, omega * C(L::w[0]), omega * C(L::w[Q - 2]), omega * C(L::w[Q - 1])};
+}
+// the same in scalar registers (omega is uniform over the wave)
+__device__ __forceinline__ double scalar(double v) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+__device__ __forceinline__ float scalar(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(unsigned, v)));
+}
+template <int Q, typename C>
+__device__ __forceinline__ Relax<Q, C> scalar(const Relax<Q, C> &r) {
+  return Relax<Q, C>{scalar(r.omega), scalar(r.keep), scalar(r.axis), scalar(r.diag), scalar(r.rest)};
 }
 
 // Population j of the cell at index `cell` of a plane-major buffer.  With
@@ -145,34 +233,82 @@ __device__ __forceinline__ ST *pop_ptr(ST *base, long long plane, int j, Idx<W64
   return const_cast<ST *>(pop_ptr<ST, W64>(static_cast<const ST *>(base), plane, j, cell));
 }
 
+// Post-collision values of a cell, handed to emit(j, value) one by one.  In
+// FP64 storage the relaxation (1 - omega) h + omega w (drho - 1.5 rho u^2 + cu
+// (3 rho + 4.5 rho cu)) takes three fused multiply-adds per population (the
+// terms in rho are formed once per weight, cu once per pair); kernels that
+// take several steps per pass over memory are bound by exactly these
+// operations.  The smaller forms keep the order and the roundings of h +
+// omega (w (drho + rho (3 cu + 4.5 cu cu - 1.5 u^2)) - h), as in moments, and
+// share what is equal for both members of a pair up to the sign.
+template <int Q, typename ST, typename E>
+__device__ __forceinline__ void collide(const typename Store<ST>::R (&h)[Q], const Moments<Q, typename Store<ST>::C> &m,
+                                        const Relax<Q, typename Store<ST>::C> &rx, typename Store<ST>::C Fx,
+                                        typename Store<ST>::C Fy, typename Store<ST>::C Fz, bool force, E emit) {
+  using L = Lat<Q>;
+  using C = typename Store<ST>::C;
+  const C omega = rx.omega;
+  const C uF = m.ux * Fx + m.uy * Fy + m.uz * Fz;
+  const C fpre = C(1) - C(0.5) * omega;
+  if constexpr (sizeof(ST) == 8) {
+    C usq = __builtin_fma(m.uy, m.uy, m.ux * m.ux);
+    if (L::D == 3 || (force && Fz != C(0))) usq = __builtin_fma(m.uz, m.uz, usq);
+    const C rest = __builtin_fma(C(-1.5) * m.rho, usq, m.drho), keep = rx.keep, oa = rx.axis, od = rx.diag;
+    const C a0 = oa * rest, a1 = oa * (C(3) * m.rho), a2 = oa * (C(4.5) * m.rho);
+    const C d0 = od * rest, d1 = od * (C(3) * m.rho), d2 = od * (C(4.5) * m.rho);
+    {
+      C out = __builtin_fma(keep, C(h[Q - 1]), rx.rest * rest);
+      if (force) out -= fpre * C(L::w[Q - 1]) * C(3) * uF;
+      emit(Q - 1, out);
+    }
+#pragma unroll
+    for (int j = 0; j < Q - 1; ++j) {
+      if (!leads<Q>(j)) continue;
+      const bool diag = L::w[j] == L::w[Q - 2];
+      const C c0 = diag ? d0 : a0, c1 = diag ? d1 : a1, c2 = diag ? d2 : a2;
+      const C cu = cdot<Q>(j, m.ux, m.uy, m.uz);
+      C p = __builtin_fma(cu, __builtin_fma(c2, cu, c1), __builtin_fma(keep, C(h[j]), c0));
+      C n = __builtin_fma(cu, __builtin_fma(c2, cu, -c1), __builtin_fma(keep, C(h[L::opp[j]]), c0));
+      if (force) {
+        const C cF = cdot<Q>(j, Fx, Fy, Fz), fw = fpre * C(L::w[j]);
+        const C fe = fw * (C(9) * cu * cF - C(3) * uF), fo = fw * C(3) * cF;
+        p += fe + fo;
+        n += fe - fo;
+      }
+      emit(j, p);
+      emit(L::opp[j], n);
+    }
+  } else {
+    const C usq = m.ux * m.ux + m.uy * m.uy + m.uz * m.uz, s = C(1.5) * usq;
+    auto one = [&](int j, C poly, C cu, C cF) {
+      const C wj = C(L::w[j]), heq = wj * (m.drho + m.rho * poly), hj = C(h[j]);
+      C out = hj + omega * (heq - hj);
+      if (force) out += fpre * wj * (C(3) * (cF - uF) + C(9) * cu * cF);
+      emit(j, out);
+    };
+    one(Q - 1, -s, C(0), C(0));
+#pragma unroll
+    for (int j = 0; j < Q - 1; ++j) {
+      if (!leads<Q>(j)) continue;
+      const C cu = cdot<Q>(j, m.ux, m.uy, m.uz), cF = cdot<Q>(j, Fx, Fy, Fz);
+      const C odd = C(3) * cu, even = C(4.5) * cu * cu;
+      one(j, even + odd - s, cu, cF);
+      one(L::opp[j], even - odd - s, -cu, -cF);
+    }
+  }
+}
+
 template <int Q, typename ST, bool NT, bool W64 = true>
 __device__ __forceinline__ void collide_store(const typename Store<ST>::R (&h)[Q], const Moments<Q, typename Store<ST>::C> &m,
                                               typename Store<ST>::C omega, typename Store<ST>::C Fx,
                                               typename Store<ST>::C Fy, typename Store<ST>::C Fz, bool force,
                                               ST *dst, long long plane, Idx<W64> cell) {
-  using L = Lat<Q>;
   using C = typename Store<ST>::C;
-  const C usq = m.ux * m.ux + m.uy * m.uy + m.uz * m.uz;
-  const C uF = m.ux * Fx + m.uy * Fy + m.uz * Fz;
-  const C fpre = C(1) - C(0.5) * omega;
-#pragma unroll
-  for (int j = 0; j < Q; ++j) {
-    C cu = 0, cF = 0;
-    if (L::cx[j] == 1) { cu += m.ux; cF += Fx; }
-    if (L::cx[j] == -1) { cu -= m.ux; cF -= Fx; }
-    if (L::cy[j] == 1) { cu += m.uy; cF += Fy; }
-    if (L::cy[j] == -1) { cu -= m.uy; cF -= Fy; }
-    if (L::cz[j] == 1) { cu += m.uz; cF += Fz; }
-    if (L::cz[j] == -1) { cu -= m.uz; cF -= Fz; }
-    const C wj = C(L::w[j]);
-    const C heq = wj * (m.drho + m.rho * (C(3) * cu + C(4.5) * cu * cu - C(1.5) * usq));
-    const C hj = C(h[j]);
-    C out = hj + omega * (heq - hj);
-    if (force) out += fpre * wj * (C(3) * (cF - uF) + C(9) * cu * cF);
+  collide<Q, ST>(h, m, relax<Q, C>(omega), Fx, Fy, Fz, force, [&](int j, C out) {
     ST *p = pop_ptr<ST, W64>(dst, plane, j, cell);
     if (NT) Store<ST>::st_nt(p, out);
     else Store<ST>::st(p, out);
-  }
+  });
 }
 
 // Zou-He face (Hecht & Harting 2010 form) on shifted populations; axis and
@@ -209,7 +345,7 @@ __device__ __forceinline__ void zou_he(C (&h)[Q], int axis, int sign, bool is_ve
     C mt = 0;
 #pragma unroll
     for (int j = 0; j < Q; ++j)
-      if (cax(j, axis) == 0) mt += C(cax(j, t)) * h[j];
+      if (cax(j, axis) == 0 && cax(j, t)) mt += cax(j, t) > 0 ? h[j] : -h[j];
     N[t] = C(0.5) * mt - rho * u[t] / C(3);
   }
   C hn[Q];
@@ -221,10 +357,11 @@ __device__ __forceinline__ void zou_he(C (&h)[Q], int axis, int sign, bool is_ve
     if (!(cn < 0)) continue;
     C cu = 0, corr = 0;
 #pragma unroll
-    for (int d = 0; d < Lat<Q>::D; ++d) cu += C(cax(j, d)) * u[d];
+    for (int d = 0; d < Lat<Q>::D; ++d)
+      if (cax(j, d)) cu += cax(j, d) > 0 ? u[d] : -u[d];
 #pragma unroll
     for (int t = 0; t < Lat<Q>::D; ++t)
-      if (t != axis) corr += C(cax(j, t)) * N[t];
+      if (t != axis && cax(j, t)) corr += cax(j, t) > 0 ? N[t] : -N[t];
     hn[j] = h[L::opp[j]] + C(6.0 * L::w[j]) * rho * cu - corr;
   }
 #pragma unroll
@@ -343,13 +480,31 @@ __device__ __forceinline__ void neem_correct(const G &a, int f, typename Store<S
           bz = vel ? C(a.face[f].u[2]) : m.uz;
   const C usq1 = m.ux * m.ux + m.uy * m.uy + m.uz * m.uz;
   const C usqb = bx * bx + by * by + bz * bz;
+  if constexpr (sizeof(ST) == 8) {
+    // rb P(ub) - rho1 P(u1) has one factor: the density step on a pressure
+    // face (ub = u1), the density on a velocity face (rb = rho1), times
+    // const + 3 c.d + 4.5 (c.d) (c.s)
+    const C f1 = vel ? m.rho : rb - m.rho;
+    const C dx = vel ? bx - m.ux : m.ux, dy = vel ? by - m.uy : m.uy, dz = vel ? bz - m.uz : m.uz;
+    const C sx = vel ? bx + m.ux : m.ux, sy = vel ? by + m.uy : m.uy, sz = vel ? bz + m.uz : m.uz;
+    const C c0 = f1 * (vel ? C(-1.5) * (usqb - usq1) : C(1) - C(1.5) * usq1), c1 = C(3) * f1, c2 = C(4.5) * f1;
+    h[Q - 1] = R(__builtin_fma(C(L::w[Q - 1]), c0, C(h[Q - 1])));
 #pragma unroll
-  for (int j = 0; j < Q; ++j) {
-    const C cu1 = C(L::cx[j]) * m.ux + C(L::cy[j]) * m.uy + C(L::cz[j]) * m.uz;
-    const C cub = C(L::cx[j]) * bx + C(L::cy[j]) * by + C(L::cz[j]) * bz;
-    const C pb = C(1) + C(3) * cub + C(4.5) * cub * cub - C(1.5) * usqb;
-    const C p1 = C(1) + C(3) * cu1 + C(4.5) * cu1 * cu1 - C(1.5) * usq1;
-    h[j] = R(C(h[j]) + C(L::w[j]) * (rb * pb - m.rho * p1));
+    for (int j = 0; j < Q - 1; ++j) {
+      if (!leads<Q>(j)) continue;
+      const C cd = cdot<Q>(j, dx, dy, dz), even = __builtin_fma(c2 * cd, cdot<Q>(j, sx, sy, sz), c0), odd = c1 * cd;
+      h[j] = R(__builtin_fma(C(L::w[j]), even + odd, C(h[j])));
+      h[L::opp[j]] = R(__builtin_fma(C(L::w[j]), even - odd, C(h[L::opp[j]])));
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < Q; ++j) {
+      const C cu1 = cdot<Q>(j, m.ux, m.uy, m.uz);
+      const C cub = cdot<Q>(j, bx, by, bz);
+      const C pb = C(1) + C(3) * cub + C(4.5) * cub * cub - C(1.5) * usqb;
+      const C p1 = C(1) + C(3) * cu1 + C(4.5) * cu1 * cu1 - C(1.5) * usq1;
+      h[j] = R(C(h[j]) + C(L::w[j]) * (rb * pb - m.rho * p1));
+    }
   }
 }
 
@@ -826,7 +981,7 @@ __device__ __forceinline__ void cell_update(const G &a, int x, int y, int z, dou
             if (iy) { const int t = cy > 0 ? 2 : 3; if (g < 0 || a.face[t].prio > a.face[g].prio) g = t; }
             if (iz) { const int t = cz > 0 ? 4 : 5; if (g < 0 || a.face[t].prio > a.face[g].prio) g = t; }
             if (g != f) continue;
-            const C cu = C(cx) * uext[0] + C(cy) * uext[1] + C(cz) * uext[2];
+            const C cu = cdot<Q>(j, uext[0], uext[1], uext[2]);
             h[j] = R(-C(h[j]) + C(L::w[j]) * (p2 * (C(1) + C(4.5) * cu * cu - C(1.5) * vsq) - C(2)));
           }
         }

@@ -35,6 +35,7 @@
 #include "../../include/lbm_hip.h"
 #include "lbm_cell.h"
 #include "lbm_launch.h"
+#include "lbm_multi2d.h"
 
 namespace lbm {
 
@@ -454,6 +455,16 @@ static void dispatch_qs(int Q, int storage, Args... args) {
   }
 }
 
+template <template <typename> class F, typename... Args>
+static void dispatch_s(int storage, Args... args) {
+  switch (storage) {
+    case LBM_STORE_F32: F<float>::run(args...); break;
+    case LBM_STORE_F64: F<double>::run(args...); break;
+    case LBM_STORE_F16: F<__half>::run(args...); break;
+    case LBM_STORE_BF16: F<__hip_bfloat16>::run(args...); break;
+  }
+}
+
 template <int Q, typename ST>
 struct InitL {
   static void run(const KArgs &a, dim3 g, dim3 b, hipStream_t s, const double *r, const double *u) {
@@ -830,8 +841,52 @@ static int finalize_sums(lbm_handle *h, lbm_sums *out) {
   return LBM_OK;
 }
 
+// Plain D2Q9 steps run several per launch (k_multi2d) unless a face needs
+// more than that kernel has (multi2d_class), the forcing correction runs
+// between steps, a plane needs 64-bit offsets, or the handle was set to the
+// general path of the single-step kernel or to its LDS halo.
+static int multi2d_cls(const lbm_handle *h) {
+  if (h->Q != 9 || h->forcing || h->w64 || h->lds || !h->wave_paths) return MULTI2D_NONE;
+  return multi2d_class(h->face, h->has_flags, h->ncell, h->esize);
+}
+
+static void launch_multi2d(lbm_handle *h, const Multi2dPlan &p, int cls, int steps) {
+  Multi2dArgs a;
+  memset(&a, 0, sizeof(a));
+  a.src = h->buf[h->cur];
+  a.dst = h->buf[h->cur ^ 1];
+  a.steps = steps;
+  a.plane = h->plane;
+  a.nx = h->nx;
+  a.ny = h->ny;
+  a.px = h->px;
+  a.per[0] = h->per[0];
+  a.per[1] = h->per[1];
+  a.face = h->dface;
+  a.links = h->has_flags ? h->links : nullptr;
+  a.omega = h->omega;
+  for (int i = 0; i < 3; ++i) a.F[i] = h->F[i];
+  a.ntx = (h->nx + p.tw - 1) / p.tw;
+  a.tw = p.tw;
+  a.th = p.th;
+  a.ntiles = a.ntx * ((h->ny + p.th - 1) / p.th);
+  dispatch_s<Multi2dL>(h->storage, a, h->stream, cls, p.wide);
+  h->cur ^= 1;
+  h->steps += steps;
+}
+
 int lbm_step(lbm_handle *h, int32_t nsteps) {
   if (!h || nsteps < 0) return fail(h, LBM_EINVAL, "lbm_step: bad argument");
+  const int cls = multi2d_cls(h);
+  if (nsteps > 1 && cls != MULTI2D_NONE) {
+    const Multi2dPlan p = multi2d_plan(h->nx, h->ny, h->ncell, h->esize, cls != MULTI2D_BOX);
+    const int n = (nsteps + p.steps - 1) / p.steps;
+    for (int i = 0; i < n; ++i) {  // as even as possible
+      launch_multi2d(h, p, cls, nsteps / n + (i < nsteps % n ? 1 : 0));
+      HIPCHK(h, hipGetLastError());
+    }
+    return LBM_OK;
+  }
   for (int i = 0; i < nsteps; ++i) {
     const int rc = launch_step(h, 0);
     if (rc) return rc;

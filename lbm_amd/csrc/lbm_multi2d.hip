@@ -1,0 +1,353 @@
+// Several D2Q9 steps per launch: every block holds a tile of the domain with
+// its halo in LDS, advances it `steps` times there and writes the tile's
+// cells once.
+//
+// What bounds the single-step kernel it replaces: on small domains the
+// launch (3.5-4.5 us a step whatever the cell count), on large ones HBM (72 B
+// per FP32 cell update, every step).  Here both are paid once per `steps`
+// updates; what is left is the FP64 (FP32 for 16-bit storage) arithmetic of
+// the updates, 1.1-1.3 times as many as cells for the halo.
+//
+// In place: a step overwrites the tile's old state, so LDS holds it once.
+// The cells of a step are taken in row-major order, one per thread and
+// round; a round's new values are written, after a barrier, pitch + 2 slots
+// below their cells' old ones, which is below whatever a later round still
+// reads (its cells' neighbours one row back and, on an open x face, two
+// columns further in).  As the valid region shrinks by a row and a column
+// per step the shifted region stays within the slots it started from, except
+// along a clipped lower edge, where `pad` slots are left in front.
+//
+// The arithmetic is that of the single-step kernels, and between steps a
+// population takes its storage form, so the result equals that many single
+// steps bit for bit.
+#include "lbm_multi2d.h"
+
+#include <algorithm>
+
+namespace lbm {
+
+// Per-cell word of a domain with faces or solids: bits 0..7, the population
+// bounces back (its upstream cell is solid or across a face); WORD_RULE, the
+// cell lies on a moving wall or an open face; WORD_SOLID, no update.  Walls
+// and obstacles cost a select per load this way; the boundary code of the
+// single-step kernels, run every step by every edge wave, took 3-4 us a step.
+constexpr uint32_t WORD_RULE = 0x4000u, WORD_SOLID = 0x8000u;
+
+__device__ __forceinline__ int wrap(int c, int n) {
+  c %= n;
+  return c < 0 ? c + n : c;
+}
+
+// The face rules of a cell whose populations h are gathered and bounced back:
+// moving walls (Ladd), anti-bounce-back, Zou-He and NEEM across x.  src, word:
+// the tile, c: the cell, on: bit f set where the cell lies on face f, kind /
+// prio: the faces' in scalar registers, face: the table in LDS.
+template <typename ST, int CLS, int CAP>
+__device__ __forceinline__ void face_rules(const ST *src, const uint16_t *word, int pitch, int c, unsigned on,
+                                           const int (&kind)[4], const int (&prio)[4], const FaceDev *face,
+                                           const double *F, typename Store<ST>::R (&h)[9]) {
+  using L = Lat<9>;
+  using C = typename Store<ST>::C;
+  using R = typename Store<ST>::R;
+  // population j of a cell on the faces `at` enters across face f and f owns
+  // the crossing (the higher priority, ties to the x face)
+  auto owned = [&](int j, int f, unsigned at) {
+    const int fx = L::cx[j] > 0 ? 0 : 1, fy = L::cy[j] > 0 ? 2 : 3;
+    if (!((at >> f) & 1u) || (f < 2 ? L::cx[j] == 0 || f != fx : L::cy[j] == 0 || f != fy)) return false;
+    if (L::cx[j] == 0 || L::cy[j] == 0) return true;
+    return f < 2 ? !(((at >> fy) & 1u) && prio[fy] > prio[fx]) : !((at >> fx) & 1u) || prio[fy] > prio[fx];
+  };
+  auto ladd = [&](unsigned at, R (&v)[9]) {
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      if (kind[f] != LBM_FACE_WALL) continue;  // uniform
+      const C u0 = C(face[f].u[0]), u1 = C(face[f].u[1]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (owned(j, f, at)) v[j] = R(C(v[j]) + C(6) * C(L::w[j]) * cdot<9>(j, u0, u1, C(0)));
+    }
+  };
+  ladd(on, h);
+  if (CLS != MULTI2D_OPEN) return;
+#pragma unroll
+  for (int f = 0; f < 2; ++f) {
+    const int in = f == 0 ? 1 : -1;
+    if (kind[f] == LBM_FACE_PRESSURE_ABB) {
+      if (!((on >> f) & 1u)) continue;
+      C u1[3], u2[3], ue[3];
+      cell_velocity<9, ST>(src, CAP, c + in, F[0], F[1], F[2], u1);
+      cell_velocity<9, ST>(src, CAP, c + 2 * in, F[0], F[1], F[2], u2);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) ue[d] = C(1.5) * u1[d] - C(0.5) * u2[d];
+      const C vsq = ue[0] * ue[0] + ue[1] * ue[1] + ue[2] * ue[2];
+      const C p2 = C(2) * C(face[f].rho);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (L::cx[j] != in || !owned(j, f, on)) continue;
+        const C cu = cdot<9>(j, ue[0], ue[1], ue[2]);
+        h[j] = R(-C(h[j]) + C(L::w[j]) * (p2 * (C(1) + C(4.5) * cu * cu - C(1.5) * vsq) - C(2)));
+      }
+    } else if (kind[f] == LBM_FACE_VELOCITY_ZH || kind[f] == LBM_FACE_PRESSURE_ZH) {
+      if ((on >> f) & 1u)
+        zou_he<9, R>(h, 0, -in, kind[f] == LBM_FACE_VELOCITY_ZH, R(face[f].u[0]), R(face[f].u[1]), R(face[f].u[2]),
+                     R(face[f].rho));
+    } else if (kind[f] == LBM_FACE_PRESSURE_NEEM || kind[f] == LBM_FACE_VELOCITY_NEEM) {
+      if (!((on >> f) & 1u)) continue;
+      const int n1 = c + in;
+      const uint32_t w1 = word[n1];
+      if (w1 & WORD_SOLID) continue;  // the cell keeps its bounce-back values
+      // the inward neighbour's populations after streaming
+#pragma unroll
+      for (int j = 0; j < 9; ++j) {
+        const bool back = j < 8 && ((w1 >> j) & 1u);
+        h[j] = Store<ST>::ld(src + (back ? L::opp[j] * CAP + n1 : j * CAP + n1 - L::cx[j] - pitch * L::cy[j]));
+      }
+      ladd(on & 12u, h);
+      struct {
+        const FaceDev *face;
+        const double *F;
+      } view{face, F};
+      neem_correct<9, ST>(view, f, h);
+    }
+  }
+}
+
+template <typename ST, int CLS, int NT>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) k_multi2d(const Multi2dArgs m) {
+  using L = Lat<9>;
+  using C = typename Store<ST>::C;
+  using R = typename Store<ST>::R;
+  constexpr bool FACES = CLS != MULTI2D_BOX;
+  constexpr int CAP = multi2d_cap((int)sizeof(ST), FACES);
+  __shared__ __align__(16) ST pop[9 * CAP];
+  __shared__ uint16_t word[FACES ? CAP : 1];
+  __shared__ FaceDev face[FACES ? 4 : 1];
+  // contiguous ranges of tiles per XCD, so that tiles sharing a halo share an L2
+  constexpr int NXCD = 8;
+  const int chunk = (m.ntiles + NXCD - 1) / NXCD;
+  const int id = (int)(blockIdx.x % NXCD) * chunk + (int)(blockIdx.x / NXCD);
+  if (id >= m.ntiles || (int)(blockIdx.x / NXCD) >= chunk) return;  // uniform per block
+  const ST *src = static_cast<const ST *>(m.src);
+  ST *dst = static_cast<ST *>(m.dst);
+  const uint32_t *links = m.links;
+  const FaceDev *gface = m.face;
+  long long plane = m.plane;
+  int nx = m.nx, ny = m.ny, px = m.px, x0, y0, x1, y1;
+  bool perx = !FACES || m.per[0], pery = !FACES || m.per[1];
+  double omega_ = m.omega;
+  if (FACES && m.tiles) {
+    const MultiTile t = m.tiles[id];
+    if (!m.active[t.d]) return;
+    const DomainDev &d = m.doms[t.d];
+    src += d.pop_off;
+    dst += d.pop_off;
+    links += d.cell_off;
+    plane = d.plane;
+    nx = d.nx;
+    ny = d.ny;
+    px = d.px;
+    perx = d.per[0] != 0;
+    pery = d.per[1] != 0;
+    gface = d.face;
+    omega_ = d.omega;
+    x0 = t.x0;
+    y0 = t.y0;
+    x1 = x0 + t.w - 1;
+    y1 = y0 + t.h - 1;
+  } else {
+    x0 = (id % m.ntx) * m.tw;
+    y0 = (id / m.ntx) * m.th;
+    x1 = min(x0 + m.tw, nx) - 1;
+    y1 = min(y0 + m.th, ny) - 1;
+  }
+  const int tid = (int)threadIdx.x;
+  // face kinds and priorities in scalar registers; `rules`, faces whose cells
+  // need more than bounce-back
+  int kind[4] = {0, 0, 0, 0}, prio[4] = {0, 0, 0, 0};
+  unsigned rules = 0;
+  if (FACES) {
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      kind[f] = gface[f].kind;
+      prio[f] = gface[f].prio;
+      const bool rest = kind[f] == LBM_FACE_WALL && gface[f].u[0] == 0.0 && gface[f].u[1] == 0.0;
+      if (kind[f] != LBM_FACE_PERIODIC && !rest) rules |= 1u << f;
+    }
+    if (tid < 4) face[tid] = gface[tid];
+    __syncthreads();
+  }
+  const int T = m.steps;
+  const Extent rx = multi2d_extent(x0, x1, T, nx, perx), ry = multi2d_extent(y0, y1, T, ny, pery);
+  const int pitch = rx.hi - rx.lo + 1, rows = ry.hi - ry.lo + 1;
+  const int shift = pitch + 2;
+  int pad = 0;
+  for (int s = 1; s < T; ++s) {
+    const int lx = multi2d_extent(x0, x1, T - s, nx, perx).lo, ly = multi2d_extent(y0, y1, T - s, ny, pery).lo;
+    pad = max(pad, s * shift - (ly - ry.lo) * pitch - (lx - rx.lo));
+  }
+  // the domain's first and last cell in the tile's coordinates (beyond reach
+  // on a periodic axis)
+  const int flo0 = perx ? -1 : -rx.lo, fhi0 = perx ? -1 : nx - 1 - rx.lo, flo1 = pery ? -1 : -ry.lo,
+            fhi1 = pery ? -1 : ny - 1 - ry.lo;
+  auto faces_of = [&](int x, int y) {
+    return (x == flo0 ? 1u : 0u) | (x == fhi0 ? 2u : 0u) | (y == flo1 ? 4u : 0u) | (y == fhi1 ? 8u : 0u);
+  };
+  // row of a linear index: exact for indices below 2^13 and widths below 2^7
+  auto recip = [](int w) { return (unsigned)((1 << 20) / w + 1); };
+  {
+    const unsigned rp = recip(pitch);
+    for (int i = tid; i < rows * pitch; i += NT) {
+      const int ly = (int)(((unsigned)i * rp) >> 20), lx = i - ly * pitch;
+      int gx = rx.lo + lx, gy = ry.lo + ly;
+      if (perx) gx = wrap(gx, nx);
+      if (pery) gy = wrap(gy, ny);
+      const unsigned cell = (unsigned)gx + (unsigned)px * (unsigned)gy;
+#pragma unroll
+      for (int j = 0; j < 9; ++j) pop[j * CAP + pad + i] = src[j * plane + cell];
+      if (FACES) {
+        uint32_t w = 0;
+        if (links) {
+          const uint32_t l = links[cell];
+          w = (l & 0xffu) | ((l & LINK_SELF_SOLID) >> 16);
+        }
+        const unsigned on = faces_of(lx, ly);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (on & ((L::cx[j] > 0 ? 1u : (L::cx[j] < 0 ? 2u : 0u)) | (L::cy[j] > 0 ? 4u : (L::cy[j] < 0 ? 8u : 0u))))
+            w |= 1u << j;
+        if (on & rules) w |= WORD_RULE;
+        word[i] = (uint16_t)w;
+      }
+    }
+  }
+  const Relax<9, C> rel = scalar(relax<9, C>(C(omega_)));
+  const C Fx = C(m.F[0]), Fy = C(m.F[1]), Fz = C(m.F[2]);
+  const bool force = m.F[0] != 0.0 || m.F[1] != 0.0 || m.F[2] != 0.0;
+  for (int s = 1; s <= T; ++s) {
+    const Extent ex = multi2d_extent(x0, x1, T - s, nx, perx), ey = multi2d_extent(y0, y1, T - s, ny, pery);
+    const int w = ex.hi - ex.lo + 1, cells = w * (ey.hi - ey.lo + 1);
+    const unsigned rw = recip(w);
+    const bool last = s == T;
+    const ST *in = pop + (pad - (s - 1) * shift);
+    ST *out = pop + (pad - s * shift);
+    __syncthreads();  // the load, or the previous step's last writes
+    for (int base = 0; base < cells; base += NT) {
+      const int k = base + tid;
+      const bool here = k < cells;
+      const int ly = (int)(((unsigned)k * rw) >> 20);
+      const int x = k - ly * w + (ex.lo - rx.lo), y = ly + (ey.lo - ry.lo);
+      const int c = x + pitch * y;
+      ST f[9];
+#pragma unroll
+      for (int j = 0; j < 9; ++j) f[j] = ST(0.0f);  // a solid cell's populations stay zero
+      const uint32_t cw = FACES && here ? word[c] : 0u;
+      const bool live = here && !(cw & WORD_SOLID);
+      if (live) {
+        R h[9];
+        if (FACES && __ballot(cw != 0)) {
+#pragma unroll
+          for (int j = 0; j < 9; ++j) {
+            const bool back = j < 8 && ((cw >> j) & 1u);
+            h[j] = Store<ST>::ld(in + (back ? L::opp[j] * CAP + c : j * CAP + c - L::cx[j] - pitch * L::cy[j]));
+          }
+          if (__ballot(cw & WORD_RULE))
+            face_rules<ST, CLS, CAP>(in, word, pitch, c, faces_of(x, y), kind, prio, face, m.F, h);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 9; ++j) h[j] = Store<ST>::ld(in + j * CAP + c - L::cx[j] - pitch * L::cy[j]);
+        }
+        const Moments<9, C> mo = moments<9, C>(h, Fx, Fy, Fz);
+        collide<9, ST>(h, mo, rel, Fx, Fy, Fz, force, [&](int j, C value) { Store<ST>::st(&f[j], value); });
+      }
+      if (!last) {
+        __syncthreads();  // every read of this round is done
+        if (here)
+#pragma unroll
+          for (int j = 0; j < 9; ++j) out[j * CAP + c] = f[j];
+      } else if (live) {
+        const unsigned cell = (unsigned)(x + rx.lo) + (unsigned)px * (unsigned)(y + ry.lo);
+#pragma unroll
+        for (int j = 0; j < 9; ++j) dst[j * plane + cell] = f[j];
+      }
+    }
+  }
+}
+
+// Tiles of a power of two of cells, as square as it gets: about one per CU as
+// long as that leaves at least 64 cells and at most 4 KB per direction (512,
+// 1024 or 2048 cells), which with the halo is what two blocks of a CU hold.
+// Small tiles take 8 steps (the launch is shared by more of them), large ones
+// 6, fewer where the halo would not fit.  For a single domain the height may
+// then grow to twice that where it saves a round of blocks: 512 run at once,
+// the last 256 or fewer of them alone on their CU in about 0.65 of the time
+// (in the formula, the cells updated per block, 1.5 per cell loaded, and 1000
+// for the launch; 909 x 1366 BF16 17.8 to 13.2 us a step).
+// 1024 threads where a CU has one block anyway.
+// Where both buffers exceed the 256 MB of cache, rows of 256 bytes and fewer
+// steps: the lines of a tile's ragged edge then come from memory.
+// Best and next of a sweep over tiles of 8 x 4 to 128 x 32 cells and 2 to 12
+// steps, microseconds per step, single-step launches last:
+//   256 x 64 FP64     8 x 8, 8 steps   1.66    16 x 4, 8     1.75     4.0
+//   256 x 128 FP32    16 x 8, 8        3.62    8 x 16, 8     3.75     5.4
+//   512 x 256 FP32    32 x 16, 8       3.14    32 x 16, 6    3.11     4.7
+//   1024^2 FP32       32 x 32, 6      12.7     64 x 16, 4   13.1     17.2
+//   4096 x 2048 FP32  64 x 20, 4      86       32 x 32, 6   93      119
+//   2048^2 FP64       32 x 16, 4      55       32 x 20, 3   58      113
+//   4096 x 2048 FP16  128 x 20, 4     56       64 x 32, 6   56       81
+Multi2dPlan multi2d_plan(int nx, int ny, long long cells, int esize, bool faces) {
+  constexpr int NCU = 256;
+  constexpr long long CACHE = 256ll << 20;
+  const int cap = multi2d_cap(esize, faces), most = 4096 / esize;
+  Multi2dPlan p;
+  if (2 * 9 * esize * cells > CACHE) {
+    p.tw = std::min(256 / esize, nx);
+    p.th = std::min(24, ny);
+    p.steps = 4;
+    p.wide = false;
+    while (multi2d_slots(p.tw, p.th, p.steps) > cap) p.th -= 4;
+    return p;
+  }
+  int lg = 6;
+  while ((1 << lg) < most && ((long long)NCU << lg) < cells) ++lg;
+  p.tw = std::min(1 << (lg + 1) / 2, nx);
+  const int low = std::min(1 << lg / 2, ny), high = cells == (long long)nx * ny ? std::min(2 * low, ny) : low;
+  double least = 0.0;
+  for (int th = low; th <= high; ++th) {
+    int t = lg >= 10 ? 6 : 8;
+    while (t > 4 && multi2d_slots(p.tw, th, t) > cap) --t;
+    if (multi2d_slots(p.tw, th, t) > cap) break;
+    const long long columns = (cells + (long long)p.tw * ny - 1) / ((long long)p.tw * ny);
+    const long long tiles = columns * ((ny + th - 1) / th), rest = tiles % (2 * NCU);
+    double work = 1.5 * (p.tw + 2 * t) * (th + 2 * t);
+    for (int s = 0; s < t; ++s) work += (p.tw + 2 * s) * (th + 2 * s);
+    const double rounds = 2.0 * (double)(tiles / (2 * NCU)) + (rest == 0 ? 0.0 : rest <= NCU ? 1.3 : 2.0);
+    const double cost = (rounds * work + 1000.0) / t;
+    if (th > low && cost >= least) continue;
+    least = cost;
+    p.th = th;
+    p.steps = t;
+    p.wide = tiles <= NCU && p.tw * th >= 256;
+  }
+  return p;
+}
+
+template <typename ST, int NT>
+static void launch_multi2d(const Multi2dArgs &a, hipStream_t s, int cls) {
+  const dim3 g((unsigned)((a.ntiles + 7) / 8 * 8)), b(NT);
+  if (cls == MULTI2D_BOX) hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_BOX, NT>), g, b, 0, s, a);
+  else if (cls == MULTI2D_WALLS) hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_WALLS, NT>), g, b, 0, s, a);
+  else hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_OPEN, NT>), g, b, 0, s, a);
+}
+
+template <typename ST>
+void Multi2dL<ST>::run(const Multi2dArgs &a, hipStream_t s, int cls, bool wide) {
+  if (wide) launch_multi2d<ST, 1024>(a, s, cls);
+  else launch_multi2d<ST, 512>(a, s, cls);
+}
+
+template struct Multi2dL<float>;
+template struct Multi2dL<double>;
+template struct Multi2dL<__half>;
+template struct Multi2dL<__hip_bfloat16>;
+
+}  // namespace lbm
