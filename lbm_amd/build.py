@@ -29,7 +29,7 @@ def run(cmd, cwd=None):
 # kernels of each storage type, the warm-start network and the Poisson
 # solver (compiled in parallel)
 HIP_SOURCES = ["lbm_hip.hip", "lbm_step_f32.hip", "lbm_step_f64.hip", "lbm_step_f16.hip", "lbm_step_bf16.hip",
-               "lbm_multi2d.hip", "lbm_surrogate.hip", "lbm_poisson.hip"]
+               "lbm_multi2d.hip", "lbm_multi3d.hip", "lbm_surrogate.hip", "lbm_poisson.hip"]
 
 
 def build_hip(extra_flags=(), out=None, jobs=None):

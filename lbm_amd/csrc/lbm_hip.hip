@@ -36,6 +36,7 @@
 #include "lbm_cell.h"
 #include "lbm_launch.h"
 #include "lbm_multi2d.h"
+#include "lbm_multi3d.h"
 
 namespace lbm {
 
@@ -256,6 +257,7 @@ struct lbm_handle {
   // LBM_STEP_WAVE_PATHS=0 keeps the general path for every wave
   unsigned long long *lanes = nullptr;
   bool wave_paths = true;
+  unsigned char *solid3 = nullptr;  // blocks of k_multi3d that meet a solid
   double p_in = 1.0, p_out = 1.0;
   double *fmac = nullptr;        // (rho, u_x, u_y) of the forced cells before the correction
   long long steps = 0;
@@ -541,6 +543,58 @@ __global__ void __launch_bounds__(256) k_lanes(const uint32_t *links, int nx, in
   if ((t & 63) == 0) lanes[wave] = m;
 }
 
+static Multi3dArgs multi3d_args(const lbm_handle *h, int cls) {
+  Multi3dArgs a;
+  memset(&a, 0, sizeof(a));
+  a.plane = h->plane;
+  a.nx = h->nx;
+  a.ny = h->ny;
+  a.nz = h->nz;
+  a.px = h->px;
+  for (int i = 0; i < 3; ++i) a.per[i] = h->per[i];
+  a.face = h->dface;
+  a.links = h->has_flags ? h->links : nullptr;
+  a.solid = h->solid3;
+  a.omega = h->omega;
+  for (int i = 0; i < 3; ++i) a.F[i] = h->F[i];
+  const Multi3dPlan p = multi3d_plan(h->nx, h->ny, h->nz, h->esize, cls);
+  a.tw = p.tw;
+  a.ntx = p.ntx;
+  a.nty = p.nty;
+  a.slabs = p.slabs;
+  return a;
+}
+
+// The two-step kernel's class for this lattice, whatever paths are switched
+// off at the moment.
+static int multi3d_fit(const lbm_handle *h) {
+  // the bounce-back source's 32-bit offset spans up to four planes
+  if (h->Q != 19 || 4.0 * (double)h->plane * h->esize > 4.2e9) return MULTI3D_NONE;
+  return multi3d_class(h->face, h->has_flags, h->ncell, h->esize);
+}
+
+// The blocks of the two-step kernel that meet a solid.  Their number depends
+// on the storage form (the tile does), so the array holds the most of any.
+// Without room for it the steps run one per launch.
+static int build_solid3(lbm_handle *h) {
+  if (!h->has_flags || multi3d_fit(h) == MULTI3D_NONE) return LBM_OK;
+  if (!h->solid3) {
+    long long n = 0;
+    for (int es : {4, 8}) {
+      const Multi3dPlan p = multi3d_plan(h->nx, h->ny, h->nz, es, MULTI3D_WALLS);
+      n = std::max(n, (long long)p.ntx * p.nty * p.slabs);
+    }
+    if (hipMalloc(&h->solid3, (size_t)n) != hipSuccess) {
+      (void)hipGetLastError();
+      h->solid3 = nullptr;
+      return LBM_OK;
+    }
+  }
+  multi3d_solid(multi3d_args(h, MULTI3D_WALLS), h->solid3, h->stream);
+  HIPCHK(h, hipGetLastError());
+  return LBM_OK;
+}
+
 // (Re)build the solid-link masks and the interior lanes; they depend on the
 // periodic axes, so lbm_set_bc calls this again.
 static int build_links(lbm_handle *h) {
@@ -556,7 +610,7 @@ static int build_links(lbm_handle *h) {
                        h->nz, h->px, h->dim, h->lanes);
     HIPCHK(h, hipGetLastError());
   }
-  return LBM_OK;
+  return build_solid3(h);
 }
 
 extern "C" {
@@ -875,6 +929,12 @@ static void launch_multi2d(lbm_handle *h, const Multi2dPlan &p, int cls, int ste
   h->steps += steps;
 }
 
+// Plain D3Q19 steps run two per launch (k_multi3d) under the same conditions.
+static int multi3d_cls(const lbm_handle *h) {
+  if (h->w64 || h->lds || !h->wave_paths || (h->has_flags && !h->solid3)) return MULTI3D_NONE;
+  return multi3d_fit(h);
+}
+
 int lbm_step(lbm_handle *h, int32_t nsteps) {
   if (!h || nsteps < 0) return fail(h, LBM_EINVAL, "lbm_step: bad argument");
   const int cls = multi2d_cls(h);
@@ -886,6 +946,18 @@ int lbm_step(lbm_handle *h, int32_t nsteps) {
       HIPCHK(h, hipGetLastError());
     }
     return LBM_OK;
+  }
+  const int cls3 = multi3d_cls(h);
+  if (nsteps > 1 && cls3 != MULTI3D_NONE) {
+    Multi3dArgs a = multi3d_args(h, cls3);
+    for (; nsteps > 1; nsteps -= 2) {
+      a.src = h->buf[h->cur];
+      a.dst = h->buf[h->cur ^ 1];
+      dispatch_s<Multi3dL>(h->storage, a, h->stream, cls3);
+      HIPCHK(h, hipGetLastError());
+      h->cur ^= 1;
+      h->steps += 2;
+    }
   }
   for (int i = 0; i < nsteps; ++i) {
     const int rc = launch_step(h, 0);
@@ -1069,7 +1141,7 @@ int lbm_set_storage(lbm_handle *h, int32_t storage) {
   h->w64 = (unsigned long long)h->plane * (unsigned long long)es > 0xffffffffull;
   h->snap_last = 0;
   if (storage != LBM_STORE_F32) h->lds = false;
-  return LBM_OK;
+  return build_solid3(h);
 }
 
 int lbm_time_steps(lbm_handle *h, int32_t nsteps, double *ms) {
@@ -1198,6 +1270,7 @@ int lbm_destroy(lbm_handle *h) {
   if (h->fmac) hipFree(h->fmac);
   if (h->links) hipFree(h->links);
   if (h->lanes) hipFree(h->lanes);
+  if (h->solid3) hipFree(h->solid3);
   for (int b = 0; b < 2; ++b)
     if (h->snap[b]) hipFree(h->snap[b]);
   if (h->partials) hipFree(h->partials);

@@ -1,0 +1,76 @@
+// Two D3Q19 steps per pass over memory (k_multi3d): argument block, tile
+// geometry and the launcher.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "lbm_launch.h"
+
+namespace lbm {
+
+// What a domain's faces ask of the kernel.
+enum : int {
+  MULTI3D_BOX = 0,    // periodic, no solids
+  MULTI3D_WALLS = 1,  // bounce-back walls (resting or moving), solids; FP64 also NEEM faces across x
+  MULTI3D_NONE = -1   // anything else: one step per launch
+};
+// Threads of a block, one per (x, y) column of its region.  Two planes of 19
+// populations per column: 512 columns take 78 KB in FP32, two blocks to a CU
+// (FP64: 156 KB, one).  With walls the kernel runs at three waves per SIMD,
+// and three blocks of 256 columns run faster than one of 768 (256 x 128 x
+// 128 cavity FP32 126 against 136 us a step).
+constexpr int multi3d_threads(int esize, int cls) { return cls == MULTI3D_WALLS && esize != 8 ? 256 : 512; }
+
+// Two steps in one pass take longer than two launches (microseconds per step,
+// this kernel against single steps)
+//  - with too few columns to fill the chip: FP32 box of 64^3 9.9 against 8.6,
+//    of 128^3 49 against 59; FP32 cavity of 128 x 64 x 64 20.5 against 19.6,
+//    of 160 x 96 x 96 54 against 71; FP64 box of 40^3 6.6 against 6.7, of 52^3
+//    8.1 against 11; FP64 cavity of 50^3 15.4 against 12.2, of 97 x 61 x 45
+//    20.4 against 21.4; FP16 box of 128^3 37 against 33, of 150^3 63 against 86;
+//  - in 16-bit storage with walls, where the masks cost more than the halved
+//    traffic (512 x 128 x 128 sphere channel 187 against 181);
+//  - in FP32 with NEEM faces, whose FP64 arithmetic is done for the halo too
+//    (the same channel 289 against 249; FP64 of 300 x 200 x 101 258 against 437).
+inline int multi3d_class(const FaceDev *face, bool solids, long long cells, int esize) {
+  int c = solids ? MULTI3D_WALLS : MULTI3D_BOX;
+  for (int f = 0; f < 6; ++f) {
+    const int k = face[f].kind;
+    if (k == LBM_FACE_PERIODIC) continue;
+    if (k != LBM_FACE_WALL && !(esize == 8 && f < 2 && (k == LBM_FACE_PRESSURE_NEEM || k == LBM_FACE_VELOCITY_NEEM)))
+      return MULTI3D_NONE;
+    c = MULTI3D_WALLS;
+  }
+  const long long least = esize == 8 ? (c == MULTI3D_WALLS ? 1ll << 18 : 1ll << 17)
+                          : esize == 4 ? (c == MULTI3D_WALLS ? 3ll << 18 : 1ll << 19)
+                                       : (c == MULTI3D_WALLS ? 1ll << 62 : 3ll << 20);
+  return cells > least ? c : MULTI3D_NONE;
+}
+
+struct Multi3dArgs {
+  const void *src;
+  void *dst;
+  long long plane;
+  int nx, ny, nz, px, per[3];
+  const FaceDev *face;
+  const uint32_t *links;       // null without solids
+  const unsigned char *solid;  // per block: it reads link masks (multi3d_solid)
+  double omega, F[3];
+  // tiles of tw columns along x, nty along y and slabs along z cut evenly; a
+  // block takes one tile of one slab
+  int tw, ntx, nty, slabs;
+};
+
+struct Multi3dPlan {
+  int tw, ntx, nty, slabs;
+};
+Multi3dPlan multi3d_plan(int nx, int ny, int nz, int esize, int cls);
+
+// solid[0 .. ntx * nty * slabs) of the plan in a, from a.links
+void multi3d_solid(const Multi3dArgs &a, unsigned char *solid, hipStream_t s);
+
+template <typename ST>
+struct Multi3dL {
+  static void run(const Multi3dArgs &a, hipStream_t s, int cls);
+};
+
+}  // namespace lbm
