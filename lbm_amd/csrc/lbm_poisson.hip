@@ -5,13 +5,15 @@
 // BGK scheme (src/lbm/solver.cpp:542-545, 589-611): phi = sum_{i<Q-1} fold_i /
 // (1 - w_rest); feq_i = w_i phi, feq_rest = (w_rest - 1) phi; f = (1 - omega)
 // fold + omega feq + source * w'_i * phi for the moving populations.  Here
-// one kernel launch is one step in pull form on a structured window; the
-// cells of a face with a boundary object are rebuilt from their
-// extrapolation cell (non-equilibrium extrapolation, bnd_dirichlet.h:367-376)
-// in the same pass.  FP64 storage, unshifted populations (the reference's
-// values, ~w phi).
+// a step is in pull form on a structured window; the cells of a face with a
+// boundary object are rebuilt from their extrapolation cell (non-equilibrium
+// extrapolation, bnd_dirichlet.h:367-376) in the same pass, and a launch
+// takes several steps (k_poisson_multi).  FP64 storage, unshifted populations
+// (the reference's values, ~w phi).  The rest population is not held: nothing
+// reads it, phi being a sum over the moving ones.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -93,25 +95,89 @@ __device__ __forceinline__ bool recomputed(const PArgs &a, int f, int layer, int
   }
 }
 
-// post-streaming populations of an interior cell (all upstream cells exist)
 template <int Q>
-__device__ __forceinline__ void gather(const PArgs &a, int x, int y, double (&g)[Q]) {
-  using L = PLat<Q>;
-#pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    const long long s = (long long)(x - L::cx[i]) + (long long)a.px * (y - L::cy[i]);
-    g[i] = __builtin_nontemporal_load(&a.src[i * a.plane + s]);  // streamed once: 2.195 -> 2.076 ms at 8192^2
-  }
-}
-
-template <int Q>
-__device__ __forceinline__ double phi_of(const double (&g)[Q]) {
+__device__ __forceinline__ double phi_of(const double (&g)[Q - 1]) {
   double s = 0;
 #pragma unroll
   for (int i = 0; i < Q - 1; ++i) s += g[i];
   return (1.0 / (1.0 - PLat<Q>::w[Q - 1])) * s;
 }
 
+// Where a cell's post-streaming populations come from: an interior cell
+// gathers its own, a face cell those of its extrapolation cell (gx, gy), with
+// the rule of the boundary object it belongs to.
+struct PCell {
+  int kind;      // 0: interior, else the kind of the object
+  int face;      // the object's face
+  int gx, gy;    // cell gathered at
+  int g2x, g2y;  // Neumann: the second cell inward
+  bool fresh;    // Neumann: vars(e) is this step's phi
+};
+template <int Q>
+__device__ __forceinline__ PCell poisson_cell(const PArgs &a, int x, int y) {
+  using L = PLat<Q>;
+  PCell c = {0, 0, x, y, x, y, false};
+  if (x > 0 && x < a.nx - 1 && (L::D == 1 || (y > 0 && y < a.ny - 1))) return c;
+  // faces the cell lies on, in direction order -x +x -y +y
+  const bool on[4] = {x == 0, x == a.nx - 1, L::D == 2 && y == 0, L::D == 2 && y == a.ny - 1};
+  int prio = 0;
+#pragma unroll
+  for (int f = 0; f < 2 * L::D; ++f)
+    if (on[f] && a.kind[f] != 0 && (c.kind == 0 || a.prio[f] > prio)) {
+      c.face = f;
+      c.kind = a.kind[f];
+      prio = a.prio[f];
+    }
+  // extrapolation direction (bnd_dirichlet.h:289-312): the first missing
+  // main direction; a second one makes it the corner diagonal
+  int ed = -1;
+#pragma unroll
+  for (int d = 0; d < 2 * L::D; ++d) {
+    if (!on[d]) continue;
+    if (ed < 0) ed = d;
+    else if (ed == 0 && d == 2) ed = 6;
+    else if (ed == 0 && d == 3) ed = 7;
+    else if (ed == 1 && d == 3) ed = 4;
+    else if (ed == 1 && d == 2) ed = 5;
+  }
+  const int in = opposite_dir(ed, L::D);
+  int dx, dy;
+  dir_vec(in, dx, dy);
+  c.gx = x + dx;
+  c.gy = y + dy;
+  c.g2x = c.gx + dx;
+  c.g2y = c.gy + dy;
+#pragma unroll
+  for (int f = 0; f < 2 * L::D; ++f)
+    if (a.kind[f] && a.prio[f] < prio)
+      c.fresh = c.fresh || recomputed(a, f, 1, c.gx, c.gy, L::D) ||
+                (a.kind[f] == LBM_POISSON_NEUMANN && recomputed(a, f, 2, c.gx, c.gy, L::D));
+  return c;
+}
+
+// The rule of a face cell on its extrapolation cell's populations g (pe their
+// phi): non-equilibrium extrapolation to the boundary value pb.
+template <int Q>
+__device__ __forceinline__ void poisson_face(double pb, double pe, double (&g)[Q - 1]) {
+  using L = PLat<Q>;
+#pragma unroll
+  for (int i = 0; i < Q - 1; ++i) g[i] = L::w[i] * pb + g[i] - L::w[i] * pe;
+}
+// Neumann, zero gradient (bnd_neumann.h:50-58), from vars(e) and the
+// post-streaming phi two cells in.  vars(e) is the previous step's phi unless
+// an object applied earlier in the same step recomputed it from the
+// post-streaming populations (PCell::fresh).
+__device__ __forceinline__ double poisson_neumann(double vars_e, double phi2) { return (4.0 * vars_e - phi2 + 0.0) / 3.0; }
+
+// collision and reaction of population i
+template <int Q>
+__device__ __forceinline__ double poisson_relax(const PArgs &a, int i, double g, double phi) {
+  using L = PLat<Q>;
+  const double f = (1.0 - a.omega) * g + a.omega * (L::w[i] * phi);
+  return f + a.source * L::wp[i] * phi;
+}
+
+// One step per launch: the check steps and a call for a single step.
 template <int Q, bool CHECK>
 __global__ void __launch_bounds__(256) k_poisson_step(const PArgs a) {
   using L = PLat<Q>;
@@ -119,57 +185,27 @@ __global__ void __launch_bounds__(256) k_poisson_step(const PArgs a) {
   double red = 0;
   if (x < a.nx) {
     const long long cell = (long long)x + (long long)a.px * y;
-    // faces the cell lies on, in direction order -x +x -y +y
-    bool on[4] = {x == 0, x == a.nx - 1, L::D == 2 && y == 0, L::D == 2 && y == a.ny - 1};
-    int ff = -1;
+    auto gather = [&](int gx, int gy, double (&v)[Q - 1]) {
 #pragma unroll
-    for (int f = 0; f < 2 * L::D; ++f)
-      if (on[f] && a.kind[f] != 0 && (ff < 0 || a.prio[f] > a.prio[ff])) ff = f;
-    double g[Q];
-    if (ff < 0) {
-      gather<Q>(a, x, y, g);
-    } else {
-      // extrapolation direction (bnd_dirichlet.h:289-312): the first missing
-      // main direction; a second one makes it the corner diagonal
-      int ed = -1;
-#pragma unroll
-      for (int d = 0; d < 2 * L::D; ++d) {
-        if (!on[d]) continue;
-        if (ed < 0) ed = d;
-        else if (ed == 0 && d == 2) ed = 6;
-        else if (ed == 0 && d == 3) ed = 7;
-        else if (ed == 1 && d == 3) ed = 4;
-        else if (ed == 1 && d == 2) ed = 5;
+      for (int i = 0; i < Q - 1; ++i) {
+        const long long s = (long long)(gx - L::cx[i]) + (long long)a.px * (gy - L::cy[i]);
+        v[i] = __builtin_nontemporal_load(&a.src[i * a.plane + s]);  // streamed once: 2.195 -> 2.076 ms at 8192^2
       }
-      const int in = opposite_dir(ed, L::D);
-      int dx, dy;
-      dir_vec(in, dx, dy);
-      const int ex = x + dx, ey = y + dy;
-      double ge[Q];
-      gather<Q>(a, ex, ey, ge);
-      const double pe = phi_of<Q>(ge);
+    };
+    const PCell c = poisson_cell<Q>(a, x, y);
+    double g[Q - 1];
+    gather(c.gx, c.gy, g);
+    if (c.kind) {
+      const double pe = phi_of<Q>(g);
       double pb;
-      if (a.kind[ff] == LBM_POISSON_DIRICHLET) {
-        pb = a.val[ff][ff < 2 ? y : x];
+      if (c.kind == LBM_POISSON_DIRICHLET) {
+        pb = a.val[c.face][c.face < 2 ? y : x];
       } else {
-        // Neumann, zero gradient (bnd_neumann.h:50-58): vars(e) and the
-        // post-streaming phi two cells in.  vars(e) is the previous step's
-        // phi unless an object applied earlier in the same step recomputed
-        // it from the post-streaming populations (then pe)
-        double g2[Q];
-        gather<Q>(a, ex + dx, ey + dy, g2);
-        bool fresh = false;
-#pragma unroll
-        for (int f = 0; f < 2 * L::D; ++f)
-          if (a.kind[f] && a.prio[f] < a.prio[ff])
-            fresh = fresh || recomputed(a, f, 1, ex, ey, L::D) ||
-                    (a.kind[f] == LBM_POISSON_NEUMANN && recomputed(a, f, 2, ex, ey, L::D));
-        const long long ecell = (long long)ex + (long long)a.px * ey;
-        pb = (4.0 * (fresh ? pe : a.phi_old[ecell]) - phi_of<Q>(g2) + 0.0) / 3.0;
+        double g2[Q - 1];
+        gather(c.g2x, c.g2y, g2);
+        pb = poisson_neumann(c.fresh ? pe : a.phi_old[(long long)c.gx + (long long)a.px * c.gy], phi_of<Q>(g2));
       }
-#pragma unroll
-      for (int i = 0; i < Q - 1; ++i) g[i] = L::w[i] * pb + ge[i] - L::w[i] * pe;
-      g[Q - 1] = (L::w[Q - 1] - 1.0) * pb + ge[Q - 1] - (L::w[Q - 1] - 1.0) * pe;
+      poisson_face<Q>(pb, pe, g);
     }
     const double phi = phi_of<Q>(g);
     if (CHECK) {
@@ -178,7 +214,7 @@ __global__ void __launch_bounds__(256) k_poisson_step(const PArgs a) {
       // object rewrote it from this step's post-streaming populations (its
       // face cells and the cells it recomputes), and varsold holds the same
       // one step earlier
-      bool touched = ff >= 0;
+      bool touched = c.kind != 0;
 #pragma unroll
       for (int f = 0; f < 2 * L::D; ++f)
         if (a.kind[f])
@@ -187,14 +223,8 @@ __global__ void __launch_bounds__(256) k_poisson_step(const PArgs a) {
       red = touched ? fabs(phi - a.phi_old[cell]) : fabs(a.phi_old[cell] - a.phi_old2[cell]);
     }
     a.phi_new[cell] = phi;
-    const double om = a.omega;
 #pragma unroll
-    for (int i = 0; i < Q; ++i) {
-      const double feq = (i == Q - 1 ? L::w[i] - 1.0 : L::w[i]) * phi;
-      double f = (1.0 - om) * g[i] + om * feq;
-      if (i < Q - 1) f += a.source * L::wp[i] * phi;
-      __builtin_nontemporal_store(f, &a.dst[i * a.plane + cell]);
-    }
+    for (int i = 0; i < Q - 1; ++i) __builtin_nontemporal_store(poisson_relax<Q>(a, i, g[i], phi), &a.dst[i * a.plane + cell]);
   }
   if (CHECK) {
     __shared__ double s[256];
@@ -205,6 +235,159 @@ __global__ void __launch_bounds__(256) k_poisson_step(const PArgs a) {
       __syncthreads();
     }
     if (threadIdx.x == 0) a.partials[blockIdx.x + (long long)gridDim.x * blockIdx.y] = s[0];
+  }
+}
+
+// Several steps per launch: a block holds a tile with its halo in LDS,
+// advances it there and writes the tile's cells once.  The step it replaces
+// was bound by the launch on small windows and by HBM on large ones, both
+// paid once per `steps` here; the arithmetic (20 FP64 operations a cell) is
+// far below either.  What bounds it now: large windows, LDS (8 reads and 8
+// writes of 8 bytes per cell and step, 2.6 times over with the halo).
+// LDS holds one state: a step's cells, at most two per thread, stay in
+// registers until every thread has read (no order of the cells to keep,
+// which the rules of a face, reaching three cells inward, would ask for).
+// On small windows one wave's chain of instructions is what is left, so a
+// thread keeps its cells, and all that does not change with the step is
+// worked out once: where it gathers, the face's rule and value, the step from
+// which the cell is no longer needed.
+constexpr int MULTI_CELLS = 1024, MULTI_THREADS = 512, MULTI_RIM = 128;
+
+struct PMulti {
+  int steps, tw, th, ntx, ntiles;
+  double *phi_prev;  // phi one step before the last, null where nothing will read it
+  int write_phi;     // phi of the last step is wanted
+};
+
+// Extent along one axis of a tile's cells [b, e] `back` steps earlier: one
+// cell more at either end, and a face cell reads up to three cells inward.
+struct PExtent {
+  int lo, hi;
+};
+__host__ __device__ inline PExtent multi_extent(int b, int e, int back, int n) {
+  if (back == 0 || n == 1) return PExtent{b, e};
+  const int lo = (b < n - 3 ? b : n - 3) - back, hi = (e > 2 ? e : 2) + back;
+  return PExtent{lo > 0 ? lo : 0, hi < n - 1 ? hi : n - 1};
+}
+
+template <int Q>
+__global__ void __launch_bounds__(MULTI_THREADS) __attribute__((amdgpu_waves_per_eu(4, 4)))
+k_poisson_multi(const PArgs a, const PMulti m) {
+  using L = PLat<Q>;
+  constexpr int NP = Q - 1, NT = MULTI_THREADS, PER = MULTI_CELLS / NT;
+  __shared__ double pop[NP * MULTI_CELLS];
+  // phi of the last two steps on the first layer inside each face
+  __shared__ double rim[2][4 * MULTI_RIM];
+  // contiguous ranges of tiles per XCD, so that tiles sharing a halo share an L2
+  const int chunk = (m.ntiles + 7) / 8, id = (int)(blockIdx.x % 8) * chunk + (int)(blockIdx.x / 8);
+  if (id >= m.ntiles) return;  // uniform per block (the grid is 8 * chunk)
+  const int x0 = (id % m.ntx) * m.tw, y0 = (id / m.ntx) * m.th;
+  const int x1 = min(x0 + m.tw, a.nx) - 1, y1 = min(y0 + m.th, a.ny) - 1;
+  const PExtent rx = multi_extent(x0, x1, m.steps, a.nx), ry = multi_extent(y0, y1, m.steps, a.ny);
+  const int pitch = rx.hi - rx.lo + 1, n = pitch * (ry.hi - ry.lo + 1), tid = (int)threadIdx.x;
+  // whether the tile and its halo hold face cells
+  const bool faces = rx.lo == 0 || rx.hi == a.nx - 1 || (L::D == 2 && (ry.lo == 0 || ry.hi == a.ny - 1));
+  // row of a linear index: exact for indices below 2^10 and widths below 2^7
+  // (D1Q3 has one row)
+  const unsigned recip = (unsigned)((1 << 20) / pitch + 1);
+  auto slot_of = [&](int x, int y) { return (x - rx.lo) + pitch * (y - ry.lo); };
+  // a first-layer cell's place in rim, -1 for the others
+  auto rim_of = [&](int x, int y) {
+    if (x == 1 || x == a.nx - 2) return (x == 1 ? 0 : MULTI_RIM) + y - ry.lo;
+    if (L::D == 2 && (y == 1 || y == a.ny - 2)) return (y == 1 ? 2 : 3) * MULTI_RIM + x - rx.lo;
+    return -1;
+  };
+  // steps before the last from which on a cell is needed along one axis
+  auto need_of = [](int x, int b, int e, int len) {
+    return x >= b && x <= e ? 0 : max(max(min(b, len - 3) - x, x - max(e, 2)), 1);
+  };
+  // per cell: need; at, its gather slot, with its place in rim plus one in the
+  // upper half; rule, 0 or the second cell's slot, 1 Dirichlet / 2 Neumann on
+  // this step's phi / 3 on the last one's, and the extrapolation cell's place
+  // in rim; val, the Dirichlet value or the extrapolation cell's phi one step
+  // before the first
+  int need[PER], at[PER], rule[PER] = {};
+  double val[PER] = {};
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = tid + k * NT;
+    need[k] = m.steps;
+    if (i >= n) continue;
+    const int ly = L::D == 1 ? 0 : (int)(((unsigned)i * recip) >> 20), x = rx.lo + i - ly * pitch, y = ry.lo + ly;
+    const long long cell = (long long)x + (long long)a.px * y;
+#pragma unroll
+    for (int j = 0; j < NP; ++j) pop[j * MULTI_CELLS + i] = a.src[j * a.plane + cell];
+    at[k] = i;
+    need[k] = max(need_of(x, x0, x1, a.nx), L::D == 1 ? 0 : need_of(y, y0, y1, a.ny));
+    if (!faces) continue;  // uniform
+    const PCell c = poisson_cell<Q>(a, x, y);
+    if (c.kind && need[k] < m.steps) {
+      at[k] = slot_of(c.gx, c.gy);
+      const bool fixed = c.kind == LBM_POISSON_DIRICHLET;
+      rule[k] = slot_of(c.g2x, c.g2y) | (fixed ? 1 : c.fresh ? 2 : 3) << 12 | rim_of(c.gx, c.gy) << 16;
+      val[k] = fixed ? a.val[c.face][c.face < 2 ? y : x] : a.phi_old[(long long)c.gx + (long long)a.px * c.gy];
+    }
+    at[k] |= (rim_of(x, y) + 1) << 16;
+  }
+  __syncthreads();
+  for (int back = m.steps - 1;; --back) {
+    double f[PER][NP], phi[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      if (back < need[k]) continue;
+      auto gather = [&](int slot, double (&v)[NP]) {
+        // opaque: the compiler otherwise keeps every population's address over
+        // the steps, 40 registers
+        asm volatile("" : "+v"(slot));
+        const double *row[3] = {pop + slot - pitch - 1, pop + slot - 1, pop + slot + pitch - 1};
+#pragma unroll
+        for (int j = 0; j < NP; ++j) v[j] = row[1 - L::cy[j]][j * MULTI_CELLS + 1 - L::cx[j]];
+      };
+      gather(at[k] & 0xffff, f[k]);
+      phi[k] = phi_of<Q>(f[k]);
+      if (rule[k]) {
+        const double pe = phi[k];
+        const int kind = (rule[k] >> 12) & 15;
+        double pb = val[k];
+        if (kind > 1) {
+          double g2[NP];
+          gather(rule[k] & 0xfff, g2);
+          const double before = back == m.steps - 1 ? val[k] : rim[back & 1][rule[k] >> 16];
+          pb = poisson_neumann(kind == 2 ? pe : before, phi_of<Q>(g2));
+        }
+        poisson_face<Q>(pb, pe, f[k]);
+        phi[k] = phi_of<Q>(f[k]);
+      }
+#pragma unroll
+      for (int j = 0; j < NP; ++j) f[k][j] = poisson_relax<Q>(a, j, f[k][j], phi[k]);
+    }
+    if (back > 0) {
+      __syncthreads();  // every read of this step is done
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        if (back < need[k]) continue;
+#pragma unroll
+        for (int j = 0; j < NP; ++j) pop[j * MULTI_CELLS + tid + k * NT] = f[k][j];
+        if (at[k] >> 16) rim[(back & 1) ^ 1][(at[k] >> 16) - 1] = phi[k];
+      }
+    }
+    if (back == 0 || (back == 1 && m.phi_prev)) {
+#pragma unroll
+      for (int k = 0; k < PER; ++k) {
+        if (need[k] != 0) continue;
+        const int i = tid + k * NT, ly = L::D == 1 ? 0 : (int)(((unsigned)i * recip) >> 20);
+        const long long cell = (long long)(rx.lo + i - ly * pitch) + (long long)a.px * (ry.lo + ly);
+        if (back == 1) {
+          m.phi_prev[cell] = phi[k];
+          continue;
+        }
+#pragma unroll
+        for (int j = 0; j < NP; ++j) __builtin_nontemporal_store(f[k][j], &a.dst[j * a.plane + cell]);
+        if (m.write_phi) a.phi_new[cell] = phi[k];
+      }
+      if (back == 0) return;
+    }
+    __syncthreads();
   }
 }
 
@@ -220,19 +403,13 @@ __global__ void __launch_bounds__(256) k_poisson_init(const PArgs a, const doubl
   const long long cell = (long long)x + (long long)a.px * y;
   const double p0 = phi0[x + (long long)a.nx * y];
   vars0[cell] = p0;
-  double g[Q];
+  double g[Q - 1];
 #pragma unroll
-  for (int i = 0; i < Q; ++i) g[i] = (i == Q - 1 ? L::w[i] - 1.0 : L::w[i]) * p0;
+  for (int i = 0; i < Q - 1; ++i) g[i] = L::w[i] * p0;
   const double phi = phi_of<Q>(g);
   a.phi_new[cell] = phi;
-  const double om = a.omega;
 #pragma unroll
-  for (int i = 0; i < Q; ++i) {
-    const double feq = (i == Q - 1 ? L::w[i] - 1.0 : L::w[i]) * phi;
-    double f = (1.0 - om) * g[i] + om * feq;
-    if (i < Q - 1) f += a.source * L::wp[i] * phi;
-    a.dst[i * a.plane + cell] = f;
-  }
+  for (int i = 0; i < Q - 1; ++i) a.dst[i * a.plane + cell] = poisson_relax<Q>(a, i, g[i], phi);
 }
 
 // fixed-order sum of the block partials
@@ -325,6 +502,64 @@ static void launch_step(lbm_poisson *h) {
   h->pcur = (h->pcur + 1) % 3;
 }
 
+// Tiles of a power of two of cells, about one per CU (two at most of 32 x 16)
+// and at least 64 cells; windows beyond that take 16 x 24 cells and 6 steps,
+// the best of what 1024 cells hold with the halo.  Microseconds per step, next
+// best of a sweep and one step per launch last:
+//   D2Q5 128^2    8 x 8, 8 steps    1.07   16 x 4, 8    1.11     4.3
+//   D2Q9 200x150  16 x 8, 8         1.65   8 x 16, 8    1.55     5.7
+//   D2Q9 512^2    32 x 16, 4        3.6    16 x 32, 4   3.7      9.9
+//   D2Q9 4096^2   16 x 24, 6        156    32 x 16, 4   176      489
+//   D1Q3 100000   512, 48           0.64   512, 16      0.75     4.7
+static PMulti multi_plan(const lbm_poisson *h) {
+  constexpr int NCU = 256;
+  const long long cells = (long long)h->nx * h->ny;
+  PMulti m;
+  memset(&m, 0, sizeof(m));
+  int lg = 6;
+  while (lg < 9 && ((long long)NCU << lg) < cells) ++lg;
+  if (h->Q == 3) {
+    m.tw = std::min(1 << lg, h->nx);
+    m.th = 1;
+    m.steps = 48;
+  } else if (cells > 2ll * NCU << 9) {
+    m.tw = std::min(16, h->nx);
+    m.th = std::min(24, h->ny);
+    m.steps = 6;
+  } else {
+    m.tw = std::min(1 << (lg + 1) / 2, h->nx);
+    m.th = std::min(1 << lg / 2, h->ny);
+    m.steps = lg < 9 ? 8 : 4;
+  }
+  m.ntx = (h->nx + m.tw - 1) / m.tw;
+  m.ntiles = m.ntx * ((h->ny + m.th - 1) / m.th);
+  return m;
+}
+
+// nsteps > 1 plain steps, split evenly over the launches.  The last two
+// states of phi go to the two slots that the next step reads and the one
+// after it.
+static void launch_multi(lbm_poisson *h, int nsteps) {
+  PMulti m = multi_plan(h);
+  const int n = (nsteps + m.steps - 1) / m.steps;
+  bool neumann = false;
+  for (int f = 0; f < 4; ++f) neumann = neumann || h->kind[f] == LBM_POISSON_NEUMANN;
+  const dim3 g((m.ntiles + 7) / 8 * 8), b(MULTI_THREADS);
+  for (int i = 0; i < n; ++i) {
+    const bool last = i == n - 1;
+    m.steps = nsteps / n + (i < nsteps % n ? 1 : 0);
+    PArgs a = pargs(h);
+    a.phi_new = h->phi[(h->pcur + 2) % 3];
+    m.phi_prev = last ? h->phi[(h->pcur + 1) % 3] : nullptr;
+    m.write_phi = last || neumann;
+    if (h->Q == 3) hipLaunchKernelGGL(k_poisson_multi<3>, g, b, 0, h->stream, a, m);
+    else if (h->Q == 5) hipLaunchKernelGGL(k_poisson_multi<5>, g, b, 0, h->stream, a, m);
+    else hipLaunchKernelGGL(k_poisson_multi<9>, g, b, 0, h->stream, a, m);
+    h->cur ^= 1;
+    h->pcur = (h->pcur + 2) % 3;
+  }
+}
+
 extern "C" {
 
 int lbm_poisson_create(const lbm_poisson_params *p, lbm_poisson **out) {
@@ -350,7 +585,7 @@ int lbm_poisson_create(const lbm_poisson_params *p, lbm_poisson **out) {
     return code;
   };
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) return bail(LBM_EHIP, "lbm_poisson_create: stream");
-  const size_t pb = (size_t)h->plane * h->Q * sizeof(double);
+  const size_t pb = (size_t)h->plane * (h->Q - 1) * sizeof(double);
   for (int k = 0; k < 2; ++k) {
     if (hipMalloc(&h->buf[k], pb) != hipSuccess) return bail(LBM_ENOMEM, "lbm_poisson_create: device memory");
     if (hipMemset(h->buf[k], 0, pb) != hipSuccess) return bail(LBM_EHIP, "lbm_poisson_create: memset");
@@ -427,7 +662,8 @@ int lbm_poisson_init(lbm_poisson *h, const double *phi0) {
 int lbm_poisson_step(lbm_poisson *h, int32_t nsteps) {
   if (!h || nsteps < 0) return pfail(h, LBM_EINVAL, "lbm_poisson_step: bad argument");
   if (!h->ready) return pfail(h, LBM_EINVAL, "lbm_poisson_step: lbm_poisson_init first");
-  for (int i = 0; i < nsteps; ++i) launch_step<false>(h);
+  if (nsteps == 1) launch_step<false>(h);
+  if (nsteps > 1) launch_multi(h, nsteps);
   PCHK(h, hipGetLastError());
   return LBM_OK;
 }
