@@ -37,6 +37,7 @@
 #include "lbm_launch.h"
 #include "lbm_multi2d.h"
 #include "lbm_multi3d.h"
+#include "lbm_readback.h"
 
 namespace lbm {
 
@@ -257,6 +258,7 @@ struct lbm_handle {
   // LBM_STEP_WAVE_PATHS=0 keeps the general path for every wave
   unsigned long long *lanes = nullptr;
   bool wave_paths = true;
+  Readback out;  // staging of the read-backs
   unsigned char *solid3 = nullptr;  // blocks of k_multi3d that meet a solid
   double p_in = 1.0, p_out = 1.0;
   double *fmac = nullptr;        // (rho, u_x, u_y) of the forced cells before the correction
@@ -1045,9 +1047,7 @@ int lbm_get_macros(lbm_handle *h, double *rho, double *u) {
                        (const double *)h->fmac, h->nx, h->ny, rd, ud);
     HIPCHK(h, hipGetLastError());
   }
-  HIPCHK(h, hipMemcpyAsync(rho, rd, h->ncell * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipMemcpyAsync(u, ud, h->ncell * h->dim * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  HIPCHK(h, h->out.copy(rho, h->ncell * sizeof(double), u, h->ncell * h->dim * sizeof(double), rd, h->stream));
   return LBM_OK;
 }
 
@@ -1082,8 +1082,7 @@ int lbm_get_populations(lbm_handle *h, double *f) {
   launch_dims(h, g, b);
   dispatch_qs<GetL>(h->Q, h->storage, a, g, b, h->stream, static_cast<double *>(fd.p));
   HIPCHK(h, hipGetLastError());
-  HIPCHK(h, hipMemcpyAsync(f, fd.p, bytes, hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  HIPCHK(h, h->out.copy(f, fd.p, bytes, h->stream));
   return LBM_OK;
 }
 

@@ -21,6 +21,7 @@
 
 #include "../../include/lbm_hip.h"
 #include "../../include/lbm_poisson.h"
+#include "lbm_readback.h"
 
 namespace lbmp {
 
@@ -447,6 +448,7 @@ struct lbm_poisson {
   int kind[4] = {0, 0, 0, 0}, prio[4] = {0, 0, 0, 0};
   double *val[4] = {nullptr, nullptr, nullptr, nullptr};
   double *partials = nullptr, *sum = nullptr, *io = nullptr;
+  lbm::Readback out;  // staging of the read-backs
   bool faces_set = false, ready = false;
   hipStream_t stream = nullptr;
   std::string err;
@@ -687,8 +689,7 @@ int lbm_poisson_get(lbm_poisson *h, double *phi) {
   hipLaunchKernelGGL(k_poisson_compact, pgrid(h), dim3(256), 0, h->stream, (const double *)h->phi[h->pcur], h->nx, h->ny,
                      h->px, h->io);
   PCHK(h, hipGetLastError());
-  PCHK(h, hipMemcpyAsync(phi, h->io, (size_t)h->nx * h->ny * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-  PCHK(h, hipStreamSynchronize(h->stream));
+  PCHK(h, h->out.copy(phi, h->io, (size_t)h->nx * h->ny * sizeof(double), h->stream));
   return LBM_OK;
 }
 
