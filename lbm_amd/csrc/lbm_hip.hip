@@ -258,7 +258,8 @@ struct lbm_handle {
   // LBM_STEP_WAVE_PATHS=0 keeps the general path for every wave
   unsigned long long *lanes = nullptr;
   bool wave_paths = true;
-  Readback out;  // staging of the read-backs
+  Readback out;                     // staging of the read-backs
+  Multi3dPlan plan3{};              // tiles of k_multi3d (build_solid3)
   unsigned char *solid3 = nullptr;  // blocks of k_multi3d that meet a solid
   double p_in = 1.0, p_out = 1.0;
   double *fmac = nullptr;        // (rho, u_x, u_y) of the forced cells before the correction
@@ -545,7 +546,7 @@ __global__ void __launch_bounds__(256) k_lanes(const uint32_t *links, int nx, in
   if ((t & 63) == 0) lanes[wave] = m;
 }
 
-static Multi3dArgs multi3d_args(const lbm_handle *h, int cls) {
+static Multi3dArgs multi3d_args(const lbm_handle *h) {
   Multi3dArgs a;
   memset(&a, 0, sizeof(a));
   a.plane = h->plane;
@@ -559,7 +560,7 @@ static Multi3dArgs multi3d_args(const lbm_handle *h, int cls) {
   a.solid = h->solid3;
   a.omega = h->omega;
   for (int i = 0; i < 3; ++i) a.F[i] = h->F[i];
-  const Multi3dPlan p = multi3d_plan(h->nx, h->ny, h->nz, h->esize, cls);
+  const Multi3dPlan &p = h->plan3;
   a.tw = p.tw;
   a.ntx = p.ntx;
   a.nty = p.nty;
@@ -575,11 +576,14 @@ static int multi3d_fit(const lbm_handle *h) {
   return multi3d_class(h->face, h->has_flags, h->ncell, h->esize);
 }
 
-// The blocks of the two-step kernel that meet a solid.  Their number depends
-// on the storage form (the tile does), so the array holds the most of any.
-// Without room for it the steps run one per launch.
+// The two-step kernel's tiles, and its blocks that meet a solid.  Their number
+// depends on the storage form (the tile does), so the array holds the most of
+// any.  Without room for it the steps run one per launch.
 static int build_solid3(lbm_handle *h) {
-  if (!h->has_flags || multi3d_fit(h) == MULTI3D_NONE) return LBM_OK;
+  const int cls = multi3d_fit(h);
+  if (cls == MULTI3D_NONE) return LBM_OK;
+  h->plan3 = multi3d_plan(h->nx, h->ny, h->nz, h->esize, cls);
+  if (!h->has_flags) return LBM_OK;
   if (!h->solid3) {
     long long n = 0;
     for (int es : {4, 8}) {
@@ -592,7 +596,7 @@ static int build_solid3(lbm_handle *h) {
       return LBM_OK;
     }
   }
-  multi3d_solid(multi3d_args(h, MULTI3D_WALLS), h->solid3, h->stream);
+  multi3d_solid(multi3d_args(h), h->solid3, h->stream);
   HIPCHK(h, hipGetLastError());
   return LBM_OK;
 }
@@ -951,7 +955,7 @@ int lbm_step(lbm_handle *h, int32_t nsteps) {
   }
   const int cls3 = multi3d_cls(h);
   if (nsteps > 1 && cls3 != MULTI3D_NONE) {
-    Multi3dArgs a = multi3d_args(h, cls3);
+    Multi3dArgs a = multi3d_args(h);
     for (; nsteps > 1; nsteps -= 2) {
       a.src = h->buf[h->cur];
       a.dst = h->buf[h->cur ^ 1];

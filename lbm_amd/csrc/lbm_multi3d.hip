@@ -371,27 +371,39 @@ __attribute__((amdgpu_waves_per_eu(sizeof(ST) == 8 ? 2 : (CLS == MULTI3D_BOX ? 4
 //   256 x 192 x 160 FP16 box    8 slabs 102                   single 116
 // More than 32 planes per slab lose once a CU runs its blocks in turns (256^3
 // in 3 slabs: 377), so those are left out.
+// FP64 domains that fit the 256 MB of cache also try equal tiles of other
+// widths: 97 columns in three tiles of 32 and one of 1 waste a quarter of the
+// blocks (97 x 61 x 45 cavity 20.4 us a step, five tiles of 20 18.5; 400 x 40 x
+// 24 23.4 and 19.9).  Rows that don't start on whole lines cost 15 to 20 % (200
+// x 64 x 64 in 25 columns 50 against 42), more in the smaller storage forms,
+// so the formula has to promise a fifth.
 Multi3dPlan multi3d_plan(int nx, int ny, int nz, int esize, int cls) {
   constexpr int NCU = 256;
-  const int nt = multi3d_threads(esize, cls);
+  constexpr long long CACHE = 256ll << 20;
+  const int nt = multi3d_threads(esize, cls), line = esize == 2 ? 64 : 32;
   const int held = esize == 8 ? 1 : nt == 256 ? 3 : 2;  // blocks a CU holds
-  Multi3dPlan p;
-  p.tw = std::min(esize == 2 ? 64 : 32, nx);
-  p.ntx = (nx + p.tw - 1) / p.tw;
-  const int rh = nt / (p.tw + 2) - 2;  // tw * rh <= nt as well
-  p.nty = (ny + rh - 1) / rh;
-  p.slabs = 1;
+  Multi3dPlan best{};
   double least = 0.0;
-  for (int s = 1; s <= std::min(32 + nz / 32, nz / 2); ++s) {
-    const long long k = ((long long)p.ntx * p.nty * s + NCU - 1) / NCU;
-    if (k > held && nz > 32 * s) continue;
-    const double cost = (double)k * ((double)nz / s + 1.0) * (k < held ? 1.4 : 1.0);
-    if (least == 0.0 || cost < least) {
-      least = cost;
-      p.slabs = s;
+  auto width = [&](int tw) {
+    Multi3dPlan p;
+    p.tw = std::min(tw, nx);
+    p.ntx = (nx + p.tw - 1) / p.tw;
+    const int rh = nt / (p.tw + 2) - 2;  // tw * rh <= nt as well
+    p.nty = (ny + rh - 1) / rh;
+    for (p.slabs = 1; p.slabs <= std::max(1, std::min(32 + nz / 32, nz / 2)); ++p.slabs) {
+      const long long k = ((long long)p.ntx * p.nty * p.slabs + NCU - 1) / NCU;
+      if (k > held && nz > 32 * p.slabs) continue;
+      const double cost = (double)k * ((double)nz / p.slabs + 1.0) * (k < held ? 1.4 : 1.0);
+      if (least == 0.0 || cost < (p.tw == best.tw ? 1.0 : 0.8) * least) {
+        least = cost;
+        best = p;
+      }
     }
-  }
-  return p;
+  };
+  width(line);
+  if (esize == 8 && 2ll * 19 * esize * nx * ny * nz <= CACHE)
+    for (int n = (nx + 63) / 64; n <= (nx + 15) / 16; ++n) width((nx + n - 1) / n);
+  return best;
 }
 
 void multi3d_solid(const Multi3dArgs &a, unsigned char *solid, hipStream_t s) {
