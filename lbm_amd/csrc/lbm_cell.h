@@ -103,6 +103,14 @@ struct Moments {
   C drho, rho, ux, uy, uz;
 };
 
+// Body force of a kernel: none, along x, or any.  A force that is known to be
+// zero, or a component of it, saves the operations the compiler has to keep
+// for it (D2Q9 in FP32 storage: 122, 152 and 183 FP64 operations a cell).
+enum : int { FORCE_NONE = 0, FORCE_X = 1, FORCE_ANY = 2 };
+inline int force_kind(const double *F) {
+  return F[1] != 0.0 || F[2] != 0.0 ? FORCE_ANY : F[0] != 0.0 ? FORCE_X : FORCE_NONE;
+}
+
 // c_j . (x, y, z): only the terms c_j has (a product with a zero component is
 // an instruction the compiler must keep).
 template <int Q, typename C>
@@ -144,8 +152,8 @@ __device__ __forceinline__ float reciprocal(float x) {
 // smaller storage forms keep the population order: there the last bit of the
 // arithmetic now and then decides a stored bit, and a flipped one spreads
 // until the rounding errors of two orders have nothing in common.
-// FORCE false: no body force (the F arguments are not read).
-template <int Q, typename C, bool FORCE = true, typename R>
+// FORCE: which components of the body force there can be.
+template <int Q, typename C, int FORCE = FORCE_ANY, typename R>
 __device__ __forceinline__ Moments<Q, C> moments(const R (&h)[Q], C Fx, C Fy, C Fz) {
   using L = Lat<Q>;
   C drho = 0, jx = 0, jy = 0, jz = 0;
@@ -163,28 +171,33 @@ __device__ __forceinline__ Moments<Q, C> moments(const R (&h)[Q], C Fx, C Fy, C 
       if (L::cz[j]) { jz = fz ? (L::cz[j] > 0 ? d : -d) : (L::cz[j] > 0 ? jz + d : jz - d); fz = false; }
     }
   } else {
+    drho = C(h[0]);
 #pragma unroll
-    for (int j = 0; j < Q; ++j) drho += C(h[j]);
+    for (int j = 1; j < Q; ++j) drho += C(h[j]);
+    auto add = [](C &sum, bool &first, C v) {  // a first term is not added to zero
+      sum = first ? v : sum + v;
+      first = false;
+    };
+    bool fx = true, fy = true, fz = true;
 #pragma unroll
     for (int j = 0; j < Q - 1; ++j) {
-      if (L::cx[j] == 1) jx += C(h[j]);
-      if (L::cx[j] == -1) jx -= C(h[j]);
-      if (L::cy[j] == 1) jy += C(h[j]);
-      if (L::cy[j] == -1) jy -= C(h[j]);
-      if (L::cz[j] == 1) jz += C(h[j]);
-      if (L::cz[j] == -1) jz -= C(h[j]);
+      if (L::cx[j] == 1) add(jx, fx, C(h[j]));
+      if (L::cx[j] == -1) add(jx, fx, -C(h[j]));
+      if (L::cy[j] == 1) add(jy, fy, C(h[j]));
+      if (L::cy[j] == -1) add(jy, fy, -C(h[j]));
+      if (L::cz[j] == 1) add(jz, fz, C(h[j]));
+      if (L::cz[j] == -1) add(jz, fz, -C(h[j]));
     }
   }
   Moments<Q, C> m;
   m.drho = drho;
   m.rho = C(1) + drho;
   const C inv = reciprocal<PAIRS ? 2 : 3>(m.rho);
-  if (FORCE) {
-    m.ux = (jx + C(0.5) * Fx) * inv;
+  m.ux = (FORCE == FORCE_NONE ? jx : jx + C(0.5) * Fx) * inv;
+  if (FORCE == FORCE_ANY) {
     m.uy = (jy + C(0.5) * Fy) * inv;
     m.uz = (jz + C(0.5) * Fz) * inv;
   } else {
-    m.ux = jx * inv;
     m.uy = jy * inv;
     m.uz = L::D == 3 ? jz * inv : C(0);
   }
@@ -241,18 +254,19 @@ __device__ __forceinline__ ST *pop_ptr(ST *base, long long plane, int j, Idx<W64
 // operations.  The smaller forms keep the order and the roundings of h +
 // omega (w (drho + rho (3 cu + 4.5 cu cu - 1.5 u^2)) - h), as in moments, and
 // share what is equal for both members of a pair up to the sign.
-template <int Q, typename ST, typename E>
+template <int Q, typename ST, int FORCE = FORCE_ANY, typename E>
 __device__ __forceinline__ void collide(const typename Store<ST>::R (&h)[Q], const Moments<Q, typename Store<ST>::C> &m,
                                         const Relax<Q, typename Store<ST>::C> &rx, typename Store<ST>::C Fx,
                                         typename Store<ST>::C Fy, typename Store<ST>::C Fz, bool force, E emit) {
   using L = Lat<Q>;
   using C = typename Store<ST>::C;
   const C omega = rx.omega;
-  const C uF = m.ux * Fx + m.uy * Fy + m.uz * Fz;
+  if (FORCE == FORCE_NONE) force = false;
+  const C uF = !force ? C(0) : FORCE == FORCE_X ? m.ux * Fx : m.ux * Fx + m.uy * Fy + m.uz * Fz;
   const C fpre = C(1) - C(0.5) * omega;
   if constexpr (sizeof(ST) == 8) {
     C usq = __builtin_fma(m.uy, m.uy, m.ux * m.ux);
-    if (L::D == 3 || (force && Fz != C(0))) usq = __builtin_fma(m.uz, m.uz, usq);
+    if (L::D == 3 || (FORCE == FORCE_ANY && force && Fz != C(0))) usq = __builtin_fma(m.uz, m.uz, usq);
     const C rest = __builtin_fma(C(-1.5) * m.rho, usq, m.drho), keep = rx.keep, oa = rx.axis, od = rx.diag;
     const C a0 = oa * rest, a1 = oa * (C(3) * m.rho), a2 = oa * (C(4.5) * m.rho);
     const C d0 = od * rest, d1 = od * (C(3) * m.rho), d2 = od * (C(4.5) * m.rho);
@@ -270,30 +284,56 @@ __device__ __forceinline__ void collide(const typename Store<ST>::R (&h)[Q], con
       C p = __builtin_fma(cu, __builtin_fma(c2, cu, c1), __builtin_fma(keep, C(h[j]), c0));
       C n = __builtin_fma(cu, __builtin_fma(c2, cu, -c1), __builtin_fma(keep, C(h[L::opp[j]]), c0));
       if (force) {
-        const C cF = cdot<Q>(j, Fx, Fy, Fz), fw = fpre * C(L::w[j]);
-        const C fe = fw * (C(9) * cu * cF - C(3) * uF), fo = fw * C(3) * cF;
-        p += fe + fo;
-        n += fe - fo;
+        const C fw = fpre * C(L::w[j]);
+        if (FORCE == FORCE_X && !L::cx[j]) {  // across the force
+          p -= fw * (C(3) * uF);
+          n -= fw * (C(3) * uF);
+        } else {
+          const C cF = FORCE == FORCE_X ? Fx : cdot<Q>(j, Fx, Fy, Fz);  // a leading c_x is +1
+          const C fe = fw * (C(9) * cu * cF - C(3) * uF), fo = fw * C(3) * cF;
+          p += fe + fo;
+          n += fe - fo;
+        }
       }
       emit(j, p);
       emit(L::opp[j], n);
     }
   } else {
-    const C usq = m.ux * m.ux + m.uy * m.uy + m.uz * m.uz, s = C(1.5) * usq;
-    auto one = [&](int j, C poly, C cu, C cF) {
-      const C wj = C(L::w[j]), heq = wj * (m.drho + m.rho * poly), hj = C(h[j]);
-      C out = hj + omega * (heq - hj);
-      if (force) out += fpre * wj * (C(3) * (cF - uF) + C(9) * cu * cF);
-      emit(j, out);
+    C usq = m.ux * m.ux + m.uy * m.uy;
+    if (L::D == 3 || FORCE == FORCE_ANY) usq = usq + m.uz * m.uz;
+    const C s = C(1.5) * usq;
+    auto relaxed = [&](int j, C poly) {
+      const C heq = C(L::w[j]) * (m.drho + m.rho * poly), hj = C(h[j]);
+      return hj + omega * (heq - hj);
     };
-    one(Q - 1, -s, C(0), C(0));
+    // the force term's first part for c_j . F = cF (FORCE_X: three values)
+    auto first = [&](C cF) { return C(3) * (cF - uF); };
+    const C f0 = force ? first(C(0)) : C(0), fp = force && FORCE == FORCE_X ? first(Fx) : C(0),
+            fn = force && FORCE == FORCE_X ? first(-Fx) : C(0);
+    {
+      C out = relaxed(Q - 1, -s);
+      if (force) out += fpre * C(L::w[Q - 1]) * f0;
+      emit(Q - 1, out);
+    }
 #pragma unroll
     for (int j = 0; j < Q - 1; ++j) {
       if (!leads<Q>(j)) continue;
-      const C cu = cdot<Q>(j, m.ux, m.uy, m.uz), cF = cdot<Q>(j, Fx, Fy, Fz);
+      const C cu = cdot<Q>(j, m.ux, m.uy, m.uz);
       const C odd = C(3) * cu, even = C(4.5) * cu * cu;
-      one(j, even + odd - s, cu, cF);
-      one(L::opp[j], even - odd - s, -cu, -cF);
+      C p = relaxed(j, even + odd - s), n = relaxed(L::opp[j], even - odd - s);
+      if (force) {
+        const C fw = fpre * C(L::w[j]);
+        if (FORCE == FORCE_X && !L::cx[j]) {  // across the force
+          p += fw * f0;
+          n += fw * f0;
+        } else {
+          const C cF = FORCE == FORCE_X ? Fx : cdot<Q>(j, Fx, Fy, Fz), second = C(9) * cu * cF;  // a leading c_x is +1
+          p += fw * ((FORCE == FORCE_X ? fp : first(cF)) + second);
+          n += fw * ((FORCE == FORCE_X ? fn : first(-cF)) + second);
+        }
+      }
+      emit(j, p);
+      emit(L::opp[j], n);
     }
   }
 }

@@ -26,7 +26,7 @@ enum : int {
 // (microseconds per step, FP32 NEEM channel of 512^2 8.1 against 7.0, of
 // 1024 x 512 12.2 against 11.6, ten BF16 NEEM channels of up to 256 x 128
 // cells 13.9 against 11.6; of 256 x 128 FP32, where the launch is what
-// counts, 3.6 against 4.9, of 2048 x 1024 31.8 against 36.6).
+// counts, 3.3 against 5.4, of 2048 x 1024 31.8 against 36.6).
 inline int multi2d_class(const FaceDev *face, bool solids, long long cells, int esize) {
   int c = solids ? MULTI2D_WALLS : MULTI2D_BOX;
   for (int f = 0; f < 4; ++f) {

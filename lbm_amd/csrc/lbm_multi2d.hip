@@ -112,7 +112,10 @@ __device__ __forceinline__ void face_rules(const ST *src, const uint16_t *word, 
   }
 }
 
-template <typename ST, int CLS, int NT>
+// On large lattices the kernel is bound by issuing its FP64 operations, so a
+// force that is not there is compiled out (FORCE): 4096 x 2048 FP32, periodic
+// without a force 87 -> 67 us a step, channel with a force along x 96 -> 86.
+template <typename ST, int CLS, int FORCE, int NT>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) k_multi2d(const Multi2dArgs m) {
   using L = Lat<9>;
   using C = typename Store<ST>::C;
@@ -222,7 +225,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
   }
   const Relax<9, C> rel = scalar(relax<9, C>(C(omega_)));
   const C Fx = C(m.F[0]), Fy = C(m.F[1]), Fz = C(m.F[2]);
-  const bool force = m.F[0] != 0.0 || m.F[1] != 0.0 || m.F[2] != 0.0;
   for (int s = 1; s <= T; ++s) {
     const Extent ex = multi2d_extent(x0, x1, T - s, nx, perx), ey = multi2d_extent(y0, y1, T - s, ny, pery);
     const int w = ex.hi - ex.lo + 1, cells = w * (ey.hi - ey.lo + 1);
@@ -256,8 +258,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 #pragma unroll
           for (int j = 0; j < 9; ++j) h[j] = Store<ST>::ld(in + j * CAP + c - L::cx[j] - pitch * L::cy[j]);
         }
-        const Moments<9, C> mo = moments<9, C>(h, Fx, Fy, Fz);
-        collide<9, ST>(h, mo, rel, Fx, Fy, Fz, force, [&](int j, C value) { Store<ST>::st(&f[j], value); });
+        const Moments<9, C> mo = moments<9, C, FORCE>(h, Fx, Fy, Fz);
+        collide<9, ST, FORCE>(h, mo, rel, Fx, Fy, Fz, true, [&](int j, C value) { Store<ST>::st(&f[j], value); });
       }
       if (!last) {
         __syncthreads();  // every read of this round is done
@@ -287,12 +289,12 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 // steps: the lines of a tile's ragged edge then come from memory.
 // Best and next of a sweep over tiles of 8 x 4 to 128 x 32 cells and 2 to 12
 // steps, microseconds per step, single-step launches last:
-//   256 x 64 FP64     8 x 8, 8 steps   1.66    16 x 4, 8     1.75     4.0
-//   256 x 128 FP32    16 x 8, 8        3.62    8 x 16, 8     3.75     5.4
-//   512 x 256 FP32    32 x 16, 8       3.14    32 x 16, 6    3.11     4.7
-//   1024^2 FP32       32 x 32, 6      12.7     64 x 16, 4   13.1     17.2
-//   4096 x 2048 FP32  64 x 20, 4      86       32 x 32, 6   93      119
-//   2048^2 FP64       32 x 16, 4      55       32 x 20, 3   58      113
+//   256 x 64 FP64     8 x 8, 8 steps   1.5     8 x 8, 6     1.6      4.1
+//   256 x 128 FP32    16 x 8, 8        3.3     16 x 8, 6    3.5      5.4
+//   512 x 256 FP32    32 x 16, 8       2.7     32 x 20, 6   3.0      4.7
+//   1024^2 FP32       32 x 32, 6      11.0     64 x 16, 4  11.5     17.2
+//   4096 x 2048 FP32  64 x 20, 4      68       32 x 32, 6   70      119
+//   2048^2 FP64       32 x 16, 4      51       32 x 20, 3   58      113
 //   4096 x 2048 FP16  128 x 20, 4     56       64 x 32, 6   56       81
 Multi2dPlan multi2d_plan(int nx, int ny, long long cells, int esize, bool faces) {
   constexpr int NCU = 256;
@@ -331,18 +333,20 @@ Multi2dPlan multi2d_plan(int nx, int ny, long long cells, int esize, bool faces)
   return p;
 }
 
-template <typename ST, int NT>
+template <typename ST, int FORCE, int NT>
 static void launch_multi2d(const Multi2dArgs &a, hipStream_t s, int cls) {
   const dim3 g((unsigned)((a.ntiles + 7) / 8 * 8)), b(NT);
-  if (cls == MULTI2D_BOX) hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_BOX, NT>), g, b, 0, s, a);
-  else if (cls == MULTI2D_WALLS) hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_WALLS, NT>), g, b, 0, s, a);
-  else hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_OPEN, NT>), g, b, 0, s, a);
+  if (cls == MULTI2D_BOX) hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_BOX, FORCE, NT>), g, b, 0, s, a);
+  else if (cls == MULTI2D_WALLS) hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_WALLS, FORCE, NT>), g, b, 0, s, a);
+  else hipLaunchKernelGGL((k_multi2d<ST, MULTI2D_OPEN, FORCE, NT>), g, b, 0, s, a);
 }
 
 template <typename ST>
 void Multi2dL<ST>::run(const Multi2dArgs &a, hipStream_t s, int cls, bool wide) {
-  if (wide) launch_multi2d<ST, 1024>(a, s, cls);
-  else launch_multi2d<ST, 512>(a, s, cls);
+  const int force = force_kind(a.F);
+  if (force == FORCE_NONE) wide ? launch_multi2d<ST, FORCE_NONE, 1024>(a, s, cls) : launch_multi2d<ST, FORCE_NONE, 512>(a, s, cls);
+  else if (force == FORCE_X) wide ? launch_multi2d<ST, FORCE_X, 1024>(a, s, cls) : launch_multi2d<ST, FORCE_X, 512>(a, s, cls);
+  else wide ? launch_multi2d<ST, FORCE_ANY, 1024>(a, s, cls) : launch_multi2d<ST, FORCE_ANY, 512>(a, s, cls);
 }
 
 template struct Multi2dL<float>;

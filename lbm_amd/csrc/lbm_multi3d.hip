@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(256) k_multi3d_solid(const Multi3dArgs m, unsi
   if (threadIdx.x == 0) solid[blockIdx.x] = (unsigned char)any;
 }
 
-template <typename ST, int CLS, bool FORCE>
+template <typename ST, int CLS, int FORCE>
 __global__ void __launch_bounds__(multi3d_threads(sizeof(ST), CLS))
 __attribute__((amdgpu_waves_per_eu(sizeof(ST) == 8 ? 2 : (CLS == MULTI3D_BOX ? 4 : 3)))) k_multi3d(const Multi3dArgs m) {
   using L = Lat<19>;
@@ -188,7 +188,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(ST) == 8 ? 2 : (CLS == MULTI3D_BOX ? 4
     return w;
   };
   const Relax<19, C> rel = scalar(relax<19, C>(C(m.omega)));
-  const C Fx = FORCE ? C(m.F[0]) : C(0), Fy = FORCE ? C(m.F[1]) : C(0), Fz = FORCE ? C(m.F[2]) : C(0);
+  const C Fx = C(m.F[0]), Fy = C(m.F[1]), Fz = C(m.F[2]);
   // the rules beyond bounce-back, on populations h of a cell with mask w in
   // plane z: the Ladd terms of moving walls and the NEEM correction
   auto rules = [&](uint32_t w, int z, R (&h)[19]) {
@@ -292,7 +292,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(ST) == 8 ? 2 : (CLS == MULTI3D_BOX ? 4
       if (WALLS && __ballot(wp != 0)) rules(wp, wrapped(p, nz), h);
       const Moments<19, C> mo = moments<19, C, FORCE>(h, Fx, Fy, Fz);
       if (std::is_same<C, double>::value) reconvert(h);
-      collide<19, ST>(h, mo, rel, Fx, Fy, Fz, FORCE, [&](int j, C value) { Store<ST>::st(&v[j], value); });
+      collide<19, ST, FORCE>(h, mo, rel, Fx, Fy, Fz, true, [&](int j, C value) { Store<ST>::st(&v[j], value); });
     }
     lds_barrier();  // the previous plane's reads of the slot are done
     if (first && mine) {
@@ -330,7 +330,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(ST) == 8 ? 2 : (CLS == MULTI3D_BOX ? 4
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       if (inner && !(WALLS && (vq & LINK_SELF_SOLID))) {
         const long long zo = (long long)wrapped(q, nz) * zs;
-        collide<19, ST>(h, mo, rel, Fx, Fy, Fz, FORCE, [&](int j, C value) {
+        collide<19, ST, FORCE>(h, mo, rel, Fx, Fy, Fz, true, [&](int j, C value) {
           const ST *base = dst + (long long)j * m.plane + zo;  // uniform
           ST out;
           Store<ST>::st(&out, value);
@@ -410,18 +410,19 @@ void multi3d_solid(const Multi3dArgs &a, unsigned char *solid, hipStream_t s) {
   hipLaunchKernelGGL(k_multi3d_solid, dim3((unsigned)(a.ntx * a.nty * a.slabs)), dim3(256), 0, s, a, solid);
 }
 
+template <typename ST, int CLS>
+static void launch_multi3d(const Multi3dArgs &a, hipStream_t s) {
+  const int n = a.ntx * a.nty * a.slabs, force = force_kind(a.F);
+  const dim3 g((unsigned)((n + 7) / 8 * 8)), b(multi3d_threads(sizeof(ST), CLS));
+  if (force == FORCE_NONE) hipLaunchKernelGGL((k_multi3d<ST, CLS, FORCE_NONE>), g, b, 0, s, a);
+  else if (force == FORCE_X) hipLaunchKernelGGL((k_multi3d<ST, CLS, FORCE_X>), g, b, 0, s, a);
+  else hipLaunchKernelGGL((k_multi3d<ST, CLS, FORCE_ANY>), g, b, 0, s, a);
+}
+
 template <typename ST>
 void Multi3dL<ST>::run(const Multi3dArgs &a, hipStream_t s, int cls) {
-  const int n = a.ntx * a.nty * a.slabs;
-  const dim3 g((unsigned)((n + 7) / 8 * 8)), b(multi3d_threads(sizeof(ST), cls));
-  const bool force = a.F[0] != 0.0 || a.F[1] != 0.0 || a.F[2] != 0.0;
-  if (cls == MULTI3D_BOX) {
-    if (force) hipLaunchKernelGGL((k_multi3d<ST, MULTI3D_BOX, true>), g, b, 0, s, a);
-    else hipLaunchKernelGGL((k_multi3d<ST, MULTI3D_BOX, false>), g, b, 0, s, a);
-  } else if constexpr (sizeof(ST) != 2) {
-    if (force) hipLaunchKernelGGL((k_multi3d<ST, MULTI3D_WALLS, true>), g, b, 0, s, a);
-    else hipLaunchKernelGGL((k_multi3d<ST, MULTI3D_WALLS, false>), g, b, 0, s, a);
-  }
+  if (cls == MULTI3D_BOX) launch_multi3d<ST, MULTI3D_BOX>(a, s);
+  else if constexpr (sizeof(ST) != 2) launch_multi3d<ST, MULTI3D_WALLS>(a, s);
 }
 
 template struct Multi3dL<float>;

@@ -64,7 +64,16 @@ def both(shape, storage, faces, steps, solid=None, omega=1.2, force=(0.0, 0.0, 0
 @pytest.mark.parametrize("faces", list(FACES))
 @pytest.mark.parametrize("shape", [(5, 5), (17, 9), (64, 16), (65, 33), (131, 70), (300, 7), (7, 300)])
 def test_multi_equals_single_steps(faces, shape):
-    a, b = both(shape, "f32", FACES[faces], (2, 9, 16, 5), force=(1e-5, 0.0, 0.0) if faces == "walls" else (0.0, 0.0, 0.0))
+    for force in ((0.0, 0.0, 0.0), (1e-5, 0.0, 0.0), (1e-5, -2e-5, 0.0)) if faces in ("walls", "periodic") else ((0.0, 0.0, 0.0),):
+        a, b = both(shape, "f32", FACES[faces], (2, 9, 16, 5), force=force)
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage", ["f64", "f16"])
+@pytest.mark.parametrize("force", [(1e-5, 0.0, 0.0), (0.0, 2e-5, 0.0)])
+def test_multi_with_a_force(storage, force):
+    a, b = both((150, 77), storage, FACES["walls"], (3, 8, 13), force=force)
     assert np.isfinite(a).all() and np.array_equal(a, b)
 
 

@@ -54,7 +54,7 @@ def both(shape, storage, faces, steps, solid=None, force=(0.0, 0.0, 0.0)):
 def test_two_steps_equal_single_steps(faces, shape):
     storage = "f64" if "neem" in faces else "f32"
     force = (1e-5, 2e-6, 0.0) if faces in ("periodic", "channel") else (0.0, 0.0, 0.0)
-    for f in {(0.0, 0.0, 0.0), force}:
+    for f in {(0.0, 0.0, 0.0), (force[0], 0.0, 0.0), force}:
         a, b = both(shape, storage, FACES[faces], (2, 5), force=f)
         assert np.isfinite(a).all() and np.array_equal(a, b)
 
