@@ -314,7 +314,7 @@ static std::vector<MultiTile> multi_tiles(lbm_batch *b) {
   if (!cells) return out;
   b->mcls = MULTI2D_WALLS;  // the kernel reads every domain's masks
   for (int d = 0; d < b->ndom; ++d) {
-    const int cls = multi2d_class(b->doms[d].face, true, cells, b->esize);
+    const int cls = multi2d_class(b->doms[d].face, true);
     if (cls == MULTI2D_NONE) return out;
     b->mcls = std::max(b->mcls, cls);
   }

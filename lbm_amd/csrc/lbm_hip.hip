@@ -907,7 +907,7 @@ static int finalize_sums(lbm_handle *h, lbm_sums *out) {
 // general path of the single-step kernel or to its LDS halo.
 static int multi2d_cls(const lbm_handle *h) {
   if (h->Q != 9 || h->forcing || h->w64 || h->lds || !h->wave_paths) return MULTI2D_NONE;
-  return multi2d_class(h->face, h->has_flags, h->ncell, h->esize);
+  return multi2d_class(h->face, h->has_flags);
 }
 
 static void launch_multi2d(lbm_handle *h, const Multi2dPlan &p, int cls, int steps) {

@@ -19,15 +19,7 @@ enum : int {
   MULTI2D_OPEN = 2,   // also Zou-He, NEEM or anti-bounce-back faces across x
   MULTI2D_NONE = -1   // anything else: one step per launch
 };
-// `cells`: of the whole launch.  FP32 and 16-bit lattices with open faces
-// between 2^17 and 2^20 cells stay at one step per launch: every wave of a
-// tile at such a face takes its rules, those tiles last twice as long as the
-// others, and there are too few tiles for a second one to fill the gap
-// (microseconds per step, FP32 NEEM channel of 512^2 8.1 against 7.0, of
-// 1024 x 512 12.2 against 11.6, ten BF16 NEEM channels of up to 256 x 128
-// cells 13.9 against 11.6; of 256 x 128 FP32, where the launch is what
-// counts, 3.3 against 5.4, of 2048 x 1024 31.8 against 36.6).
-inline int multi2d_class(const FaceDev *face, bool solids, long long cells, int esize) {
+inline int multi2d_class(const FaceDev *face, bool solids) {
   int c = solids ? MULTI2D_WALLS : MULTI2D_BOX;
   for (int f = 0; f < 4; ++f) {
     const int k = face[f].kind;
@@ -41,7 +33,7 @@ inline int multi2d_class(const FaceDev *face, bool solids, long long cells, int 
       return MULTI2D_NONE;
     }
   }
-  return c == MULTI2D_OPEN && esize < 8 && cells > 1ll << 17 && cells <= 1ll << 20 ? (int)MULTI2D_NONE : c;
+  return c;
 }
 
 // One tile of a batch: the cells [x0, x0 + w) x [y0, y0 + h) of domain d.

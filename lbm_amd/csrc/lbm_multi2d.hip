@@ -9,13 +9,14 @@
 // the updates, 1.1-1.3 times as many as cells for the halo.
 //
 // In place: a step overwrites the tile's old state, so LDS holds it once.
-// The cells of a step are taken in row-major order, one per thread and
-// round; a round's new values are written, after a barrier, pitch + 2 slots
-// below their cells' old ones, which is below whatever a later round still
-// reads (its cells' neighbours one row back and, on an open x face, two
-// columns further in).  As the valid region shrinks by a row and a column
-// per step the shifted region stays within the slots it started from, except
-// along a clipped lower edge, where `pad` slots are left in front.
+// The cells of a step are taken in the order of their slots (row-major, or by
+// columns at an open x face), one per thread and round; a round's new values
+// are written, after a barrier, a line (pitch or rows) + 2 slots below their
+// cells' old ones, two lines where a face's rules reach two lines back, which
+// is below whatever a later round still reads.  As the valid region shrinks
+// by a row and a column per step the shifted region stays within the slots it
+// started from, except along a clipped lower edge, where `pad` slots are left
+// in front.
 //
 // The arithmetic is that of the single-step kernels, and between steps a
 // population takes its storage form, so the result equals that many single
@@ -43,7 +44,7 @@ __device__ __forceinline__ int wrap(int c, int n) {
 // the tile, c: the cell, on: bit f set where the cell lies on face f, kind /
 // prio: the faces' in scalar registers, face: the table in LDS.
 template <typename ST, int CLS, int CAP>
-__device__ __forceinline__ void face_rules(const ST *src, const uint16_t *word, int pitch, int c, unsigned on,
+__device__ __forceinline__ void face_rules(const ST *src, const uint16_t *word, int sx, int sy, int c, unsigned on,
                                            const int (&kind)[4], const int (&prio)[4], const FaceDev *face,
                                            const double *F, typename Store<ST>::R (&h)[9]) {
   using L = Lat<9>;
@@ -75,8 +76,8 @@ __device__ __forceinline__ void face_rules(const ST *src, const uint16_t *word, 
     if (kind[f] == LBM_FACE_PRESSURE_ABB) {
       if (!((on >> f) & 1u)) continue;
       C u1[3], u2[3], ue[3];
-      cell_velocity<9, ST>(src, CAP, c + in, F[0], F[1], F[2], u1);
-      cell_velocity<9, ST>(src, CAP, c + 2 * in, F[0], F[1], F[2], u2);
+      cell_velocity<9, ST>(src, CAP, c + in * sx, F[0], F[1], F[2], u1);
+      cell_velocity<9, ST>(src, CAP, c + 2 * in * sx, F[0], F[1], F[2], u2);
 #pragma unroll
       for (int d = 0; d < 3; ++d) ue[d] = C(1.5) * u1[d] - C(0.5) * u2[d];
       const C vsq = ue[0] * ue[0] + ue[1] * ue[1] + ue[2] * ue[2];
@@ -93,14 +94,14 @@ __device__ __forceinline__ void face_rules(const ST *src, const uint16_t *word, 
                      R(face[f].rho));
     } else if (kind[f] == LBM_FACE_PRESSURE_NEEM || kind[f] == LBM_FACE_VELOCITY_NEEM) {
       if (!((on >> f) & 1u)) continue;
-      const int n1 = c + in;
+      const int n1 = c + in * sx;
       const uint32_t w1 = word[n1];
       if (w1 & WORD_SOLID) continue;  // the cell keeps its bounce-back values
       // the inward neighbour's populations after streaming
 #pragma unroll
       for (int j = 0; j < 9; ++j) {
         const bool back = j < 8 && ((w1 >> j) & 1u);
-        h[j] = Store<ST>::ld(src + (back ? L::opp[j] * CAP + n1 : j * CAP + n1 - L::cx[j] - pitch * L::cy[j]));
+        h[j] = Store<ST>::ld(src + (back ? L::opp[j] * CAP + n1 : j * CAP + n1 - sx * L::cx[j] - sy * L::cy[j]));
       }
       ladd(on & 12u, h);
       struct {
@@ -182,11 +183,21 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
   const int T = m.steps;
   const Extent rx = multi2d_extent(x0, x1, T, nx, perx), ry = multi2d_extent(y0, y1, T, ny, pery);
   const int pitch = rx.hi - rx.lo + 1, rows = ry.hi - ry.lo + 1;
-  const int shift = pitch + 2;
+  // Tiles at an open x face go column by column, in LDS and in the order of
+  // the cells: the face's rules, as long as the rest of the update, are then
+  // taken by the wave that holds the column and not by every wave (NEEM
+  // channel of 256 x 128 FP32 3.3 -> 2.85 us a step, of 512^2 FP64 7.7 -> 5.8,
+  // of 512^2 FP32 8.1 -> 5.5 against 7.5 with one step per launch).  A cell on
+  // the upper face reaches two columns back.
+  const bool columns = CLS == MULTI2D_OPEN && !perx && ((rx.lo == 0 && kind[0] != LBM_FACE_WALL) || (rx.hi == nx - 1 && kind[1] != LBM_FACE_WALL));
+  const int sx = columns ? rows : 1, sy = columns ? 1 : pitch;  // slots from a cell to the next
+  // slots a step's state moves down by; hx: the last column it updates
+  auto shift_of = [&](int hx) { return columns ? (hx == nx - 1 && kind[1] != LBM_FACE_WALL ? 2 : 1) * rows + 2 : pitch + 2; };
   int pad = 0;
-  for (int s = 1; s < T; ++s) {
-    const int lx = multi2d_extent(x0, x1, T - s, nx, perx).lo, ly = multi2d_extent(y0, y1, T - s, ny, pery).lo;
-    pad = max(pad, s * shift - (ly - ry.lo) * pitch - (lx - rx.lo));
+  for (int s = 1, down = 0; s < T; ++s) {
+    const Extent ex = multi2d_extent(x0, x1, T - s, nx, perx), ey = multi2d_extent(y0, y1, T - s, ny, pery);
+    down += shift_of(ex.hi);
+    pad = max(pad, down - (ey.lo - ry.lo) * sy - (ex.lo - rx.lo) * sx);
   }
   // the domain's first and last cell in the tile's coordinates (beyond reach
   // on a periodic axis)
@@ -206,7 +217,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
       if (pery) gy = wrap(gy, ny);
       const unsigned cell = (unsigned)gx + (unsigned)px * (unsigned)gy;
 #pragma unroll
-      for (int j = 0; j < 9; ++j) pop[j * CAP + pad + i] = src[j * plane + cell];
+      for (int j = 0; j < 9; ++j) pop[j * CAP + pad + lx * sx + ly * sy] = src[j * plane + cell];
       if (FACES) {
         uint32_t w = 0;
         if (links) {
@@ -219,26 +230,29 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
           if (on & ((L::cx[j] > 0 ? 1u : (L::cx[j] < 0 ? 2u : 0u)) | (L::cy[j] > 0 ? 4u : (L::cy[j] < 0 ? 8u : 0u))))
             w |= 1u << j;
         if (on & rules) w |= WORD_RULE;
-        word[i] = (uint16_t)w;
+        word[lx * sx + ly * sy] = (uint16_t)w;
       }
     }
   }
   const Relax<9, C> rel = scalar(relax<9, C>(C(omega_)));
   const C Fx = C(m.F[0]), Fy = C(m.F[1]), Fz = C(m.F[2]);
+  int at = pad;  // where the state starts
   for (int s = 1; s <= T; ++s) {
     const Extent ex = multi2d_extent(x0, x1, T - s, nx, perx), ey = multi2d_extent(y0, y1, T - s, ny, pery);
-    const int w = ex.hi - ex.lo + 1, cells = w * (ey.hi - ey.lo + 1);
-    const unsigned rw = recip(w);
+    const int w = ex.hi - ex.lo + 1, rs = ey.hi - ey.lo + 1, cells = w * rs;
+    const int line = columns ? rs : w;
+    const unsigned rl = recip(line);
     const bool last = s == T;
-    const ST *in = pop + (pad - (s - 1) * shift);
-    ST *out = pop + (pad - s * shift);
+    const ST *in = pop + at;
+    at -= shift_of(ex.hi);
+    ST *out = pop + at;  // not used in the last step
     __syncthreads();  // the load, or the previous step's last writes
     for (int base = 0; base < cells; base += NT) {
       const int k = base + tid;
       const bool here = k < cells;
-      const int ly = (int)(((unsigned)k * rw) >> 20);
-      const int x = k - ly * w + (ex.lo - rx.lo), y = ly + (ey.lo - ry.lo);
-      const int c = x + pitch * y;
+      const int q = (int)(((unsigned)k * rl) >> 20), r = k - q * line;
+      const int x = (columns ? q : r) + (ex.lo - rx.lo), y = (columns ? r : q) + (ey.lo - ry.lo);
+      const int c = x * sx + y * sy;
       ST f[9];
 #pragma unroll
       for (int j = 0; j < 9; ++j) f[j] = ST(0.0f);  // a solid cell's populations stay zero
@@ -250,13 +264,13 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 #pragma unroll
           for (int j = 0; j < 9; ++j) {
             const bool back = j < 8 && ((cw >> j) & 1u);
-            h[j] = Store<ST>::ld(in + (back ? L::opp[j] * CAP + c : j * CAP + c - L::cx[j] - pitch * L::cy[j]));
+            h[j] = Store<ST>::ld(in + (back ? L::opp[j] * CAP + c : j * CAP + c - sx * L::cx[j] - sy * L::cy[j]));
           }
           if (__ballot(cw & WORD_RULE))
-            face_rules<ST, CLS, CAP>(in, word, pitch, c, faces_of(x, y), kind, prio, face, m.F, h);
+            face_rules<ST, CLS, CAP>(in, word, sx, sy, c, faces_of(x, y), kind, prio, face, m.F, h);
         } else {
 #pragma unroll
-          for (int j = 0; j < 9; ++j) h[j] = Store<ST>::ld(in + j * CAP + c - L::cx[j] - pitch * L::cy[j]);
+          for (int j = 0; j < 9; ++j) h[j] = Store<ST>::ld(in + j * CAP + c - sx * L::cx[j] - sy * L::cy[j]);
         }
         const Moments<9, C> mo = moments<9, C, FORCE>(h, Fx, Fy, Fz);
         collide<9, ST, FORCE>(h, mo, rel, Fx, Fy, Fz, true, [&](int j, C value) { Store<ST>::st(&f[j], value); });
@@ -290,7 +304,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 // Best and next of a sweep over tiles of 8 x 4 to 128 x 32 cells and 2 to 12
 // steps, microseconds per step, single-step launches last:
 //   256 x 64 FP64     8 x 8, 8 steps   1.5     8 x 8, 6     1.6      4.1
-//   256 x 128 FP32    16 x 8, 8        3.3     16 x 8, 6    3.5      5.4
+//   256 x 128 FP32    16 x 8, 8        2.85    8 x 16, 8    2.92     5.4
 //   512 x 256 FP32    32 x 16, 8       2.7     32 x 20, 6   3.0      4.7
 //   1024^2 FP32       32 x 32, 6      11.0     64 x 16, 4  11.5     17.2
 //   4096 x 2048 FP32  64 x 20, 4      68       32 x 32, 6   70      119
