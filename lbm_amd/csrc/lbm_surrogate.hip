@@ -103,11 +103,24 @@ __device__ __forceinline__ bool group_of(long long t, long long np, unsigned gro
 // channels from co0.  Lane l holds C[mm][n] in acc[r], n = l % 32, mm = 8 (r /
 // 4) + 4 (l / 32) + r % 4.  MODE 0 goes through `ep` (the wave's 32 x 40
 // elements of LDS): two 16-byte stores per lane instead of sixteen of 2 bytes.
+// DIRECT stores from the registers (whole tiles only): k_conv_lds, where that
+// LDS costs more blocks than the stores.
 constexpr int EP_STRIDE = 40;
-template <int MODE>
+template <int MODE, bool DIRECT = false>
 __device__ __forceinline__ void conv_epilogue(const ConvArgs &a, f32x16 acc, long long pp0, long long npix, int co0,
                                               int lane, u16 *ep) {
   const int m = lane & 31, g = lane >> 5, co_ = co0 + m;
+  if (MODE == 0 && DIRECT) {
+    const float bias = a.bias[co_];
+    u16 *d = a.y + pp0 * a.co + co_;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float v = acc[r] + bias;
+      if (a.relu) v = fmaxf(v, 0.f);
+      d[(((r >> 2) << 3) + 4 * g + (r & 3)) * a.co] = f2bf(v);
+    }
+    return;
+  }
   if (MODE == 0) {
     const float bias = a.bias[co_];
 #pragma unroll
@@ -187,29 +200,39 @@ __global__ void __launch_bounds__(256) k_conv(const ConvArgs a, const int ksplit
   const int k0 = kp * nks / ksplit, k1 = (kp + 1) * nks / ksplit;
   const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   if (active && k0 < k1) {
-    // the loader's step: its tap and channel, and this lane's pixel there
-    int kl = k0, tap = k0 / cpt, c = (k0 - tap * cpt) << 4;
-    const u16 *pa = nullptr, *ps = nullptr;
+    // the loader: K runs over the taps, and per tap over the upsampled and
+    // the same-level channels; it keeps this lane's address in the present run
+    // and the steps left in it
+    int kl = k0, tap = k0 / cpt, c = (k0 - tap * cpt) << 4, left = 0;
+    const u16 *pl = nullptr;
     bool in = false;
     const u16 *wl = a.w + ((long long)k0 * a.co + co0 + m) * 16 + 8 * g;
     auto aim = [&]() {
       const int ys = y + tap / 3 - 1, xs = x + tap % 3 - 1;
       in = pin && ys >= 0 && ys < a.h && xs >= 0 && xs < a.wd;
-      pa = a.a + (((long long)b * h2 + (ys >> 1)) * w2 + (xs >> 1)) * a.ca + 8 * g;
-      ps = a.s + (((long long)b * a.h + ys) * a.wd + xs) * a.cs - a.ca + 8 * g;
+      if (c < a.ca) {
+        pl = a.a + (((long long)b * h2 + (ys >> 1)) * w2 + (xs >> 1)) * a.ca + c + 8 * g;
+        left = (a.ca - c) >> 4;
+      } else {
+        pl = a.s + (((long long)b * a.h + ys) * a.wd + xs) * a.cs + (c - a.ca) + 8 * g;
+        left = (ci - c) >> 4;
+      }
     };
     aim();
     auto load = [&](u16x8 &av, u16x8 &bv) {
       if (kl >= k1) return;
       bv = *reinterpret_cast<const u16x8 *>(wl);
       av = zero;
-      if (in) av = *reinterpret_cast<const u16x8 *>((c < a.ca ? pa : ps) + c);
+      if (in) av = *reinterpret_cast<const u16x8 *>(pl);
       wl += (long long)a.co * 16;
+      pl += 16;
       ++kl;
       c += 16;
-      if (c == ci) {
-        c = 0;
-        ++tap;
+      if (--left == 0) {
+        if (c == ci) {
+          c = 0;
+          ++tap;
+        }
         aim();
       }
     };
@@ -242,21 +265,24 @@ __global__ void __launch_bounds__(256) k_conv(const ConvArgs a, const int ksplit
 }
 
 // The same convolution with the input staged in LDS (levels whose width is
-// a multiple of 32 and ci <= LDS_CI_MAX): a block computes 4 image rows x
-// 32 pixels x 32 output channels (blockIdx.y = output tile), one wave per
-// row.  The block first loads the 6 x 34 input pixels of its rows and their
-// one-pixel halo (zero outside the image; the upsampled channels first, read
-// at half resolution) with 16-byte loads, then every tap reads its A operand
-// from LDS, so each input element comes from HBM/L2 once per block instead
-// of once per tap.  Pixel stride in LDS: ci + 8 elements.
-// The weights run LDS_DEPTH steps ahead.
-constexpr int LDS_CI_MAX = 128, LDS_DEPTH = 4;
-constexpr size_t conv_lds_bytes(int ci) { return ((size_t)6 * 34 * (ci + 8) + 4 * 32 * EP_STRIDE) * sizeof(u16); }
-template <int MODE>
+// a multiple of 32 and 16, 32, 64, 96 or 128 input channels CI): a block
+// computes 4 image rows x 32 pixels x 32 output channels (blockIdx.y = output
+// tile), one wave per row.  The block first loads the 6 x 34 input pixels of
+// its rows and their one-pixel halo (zero outside the image; the upsampled
+// channels first, read at half resolution) with 16-byte loads, STAGE in
+// flight per thread, then every tap reads its A operand from LDS, so each
+// input element comes from HBM/L2 once per block instead of once per tap.
+// Pixel stride in LDS: CI + 8 elements.  The weights run LDS_DEPTH steps
+// ahead.
+// CI is a template parameter: with run-time channels a product was issued
+// with 40 scalar and 39 vector instructions of index arithmetic, which bounded
+// the kernel (16 x 128 x 256 pixels, 32 to 32 channels 34 us, now 24).
+constexpr int LDS_DEPTH = 4, STAGE = 4;
+template <int MODE, int CI>
 __global__ void __launch_bounds__(256) k_conv_lds(const ConvArgs a) {
-  extern __shared__ __align__(16) u16 xs[];  // [6][34][ci + 8], then the epilogue's [4][32][EP_STRIDE]
+  __shared__ __align__(16) u16 xs[6 * 34 * (CI + 8)];
+  constexpr int CST = CI + 8, CG = CI / 8, CPT = CI / 16, NKS = 9 * CPT, NE = 6 * 34 * CG;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int ci = a.ca + a.cs, cst = ci + 8;
   const int xt = a.wd >> 5, ry = (a.h + 3) >> 2;
   const int blk = blockIdx.x;
   const int x0 = (blk % xt) * 32;
@@ -266,28 +292,33 @@ __global__ void __launch_bounds__(256) k_conv_lds(const ConvArgs a) {
   const int h2 = a.h >> 1, w2 = a.wd >> 1;
   // stage rows y0-1 .. y0+4, columns x0-1 .. x0+32, 8 channels per load;
   // offsets from the uniform addresses of row y0 - 1
-  const int cg = ci >> 3;
-  const unsigned recip = (1u << 20) / (unsigned)cg + 1;  // e / cg, exact for e < 6 * 34 * 16
   const u16 *srow = a.s + ((long long)b * a.h + (y0 - 1)) * a.wd * a.cs - a.ca;
   const u16 *arow = a.a + ((long long)b * h2 + ((y0 - 1) >> 1)) * w2 * a.ca;
-  for (int e = threadIdx.x; e < 6 * 34 * cg; e += 256) {
-    const int pix = (int)(((unsigned)e * recip) >> 20);
-    const int c = (e - pix * cg) << 3;
-    const int r = pix / 34, yy = y0 - 1 + r, xx = x0 - 1 + (pix - 34 * r);
-    u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (yy >= 0 && yy < a.h && xx >= 0 && xx < a.wd) {
-      if (c < a.ca) v = *reinterpret_cast<const u16x8 *>(arow + ((((yy >> 1) - ((y0 - 1) >> 1)) * w2 + (xx >> 1)) * a.ca + c));
-      else v = *reinterpret_cast<const u16x8 *>(srow + ((r * a.wd + xx) * a.cs + c));
+#pragma unroll
+  for (int e0 = 0; e0 < NE; e0 += 256 * STAGE) {
+    u16x8 v[STAGE];
+#pragma unroll
+    for (int i = 0; i < STAGE; ++i) {
+      const int e = e0 + 256 * i + (int)threadIdx.x, pix = e / CG, c = (e % CG) * 8;
+      const int r = pix / 34, yy = y0 - 1 + r, xx = x0 - 1 + pix % 34;
+      v[i] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (e < NE && yy >= 0 && yy < a.h && xx >= 0 && xx < a.wd) {
+        if (c < a.ca) v[i] = *reinterpret_cast<const u16x8 *>(arow + ((((yy >> 1) - ((y0 - 1) >> 1)) * w2 + (xx >> 1)) * a.ca + c));
+        else v[i] = *reinterpret_cast<const u16x8 *>(srow + ((r * a.wd + xx) * a.cs + c));
+      }
     }
-    *reinterpret_cast<u16x8 *>(xs + pix * cst + c) = v;
+#pragma unroll
+    for (int i = 0; i < STAGE; ++i) {
+      const int e = e0 + 256 * i + (int)threadIdx.x;
+      if (e < NE) *reinterpret_cast<u16x8 *>(xs + (e / CG) * CST + (e % CG) * 8) = v[i];
+    }
   }
   const int m = lane & 31, g = lane >> 5;
-  const u16 *wrow = a.w + (long long)(co0 + m) * 16 + 8 * g;
+  const u16 *wl = a.w + (long long)(co0 + m) * 16 + 8 * g;
   const long long wstep = (long long)a.co * 16;  // elements per K step
-  const int cpt = ci >> 4, nks = 9 * cpt;
   u16x8 bv[LDS_DEPTH];
 #pragma unroll
-  for (int i = 0; i < LDS_DEPTH; ++i) bv[i] = *reinterpret_cast<const u16x8 *>(wrow + i * wstep);  // nks >= 9
+  for (int i = 0; i < LDS_DEPTH; ++i, wl += wstep) bv[i] = *reinterpret_cast<const u16x8 *>(wl);  // NKS >= 9
   __syncthreads();
   const int y = y0 + wave;
   if (y >= a.h) return;  // after the only barrier
@@ -295,25 +326,20 @@ __global__ void __launch_bounds__(256) k_conv_lds(const ConvArgs a) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   // pixel (y + dy, x0 + m + dx) sits at LDS row wave + 1 + dy, column m + 1 + dx
-  const u16 *at = xs + (wave * 34 + m) * cst + 8 * g;
-  int tap = 0, c = 0;
-  for (int k = 0; k < nks; k += LDS_DEPTH) {
+  const u16 *at = xs + (wave * 34 + m) * CST + 8 * g;
 #pragma unroll
-    for (int i = 0; i < LDS_DEPTH; ++i) {
-      if (k + i >= nks) break;  // uniform
-      const u16x8 av = *reinterpret_cast<const u16x8 *>(at + ((tap / 3) * 34 + tap % 3) * cst + c);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv[i]), acc,
-                                                    0, 0, 0);
-      if (k + i + LDS_DEPTH < nks) bv[i] = *reinterpret_cast<const u16x8 *>(wrow + (k + i + LDS_DEPTH) * wstep);
-      c += 16;
-      if (c == ci) {
-        c = 0;
-        ++tap;
-      }
+  for (int k = 0; k < NKS; ++k) {
+    const int tap = k / CPT, c = (k % CPT) * 16;
+    const u16x8 av = *reinterpret_cast<const u16x8 *>(at + ((tap / 3) * 34 + tap % 3) * CST + c);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av),
+                                                  __builtin_bit_cast(bf16x8, bv[k % LDS_DEPTH]), acc, 0, 0, 0);
+    if (k + LDS_DEPTH < NKS) {
+      bv[k % LDS_DEPTH] = *reinterpret_cast<const u16x8 *>(wl);
+      wl += wstep;
     }
   }
   const long long prow = ((long long)b * a.h + y) * a.wd + x0;
-  conv_epilogue<MODE>(a, acc, prow, prow + 32, co0, lane, xs + 6 * 34 * cst + wave * 32 * EP_STRIDE);
+  conv_epilogue<MODE, true>(a, acc, prow, prow + 32, co0, lane, nullptr);
 }
 
 struct WgradArgs {
@@ -1258,20 +1284,32 @@ static unsigned conv_blocks(long long npix, int co) {
   return (unsigned)((tiles + per - 1) / per);
 }
 
-// the large levels (at least 65536 pixels, width a multiple of 32, at most
-// LDS_CI_MAX input channels) run k_conv_lds
+// the large levels (at least 65536 pixels, width a multiple of 32, channels
+// that k_conv_lds is built for) run k_conv_lds
 // (16384 pixels measured the same per training step, 4096 3 % slower)
-static bool conv_lds(long long npix, int w, int ci) { return npix >= 65536 && w % 32 == 0 && ci <= LDS_CI_MAX; }
+static bool conv_lds(long long npix, int w, int ci) {
+  return npix >= 65536 && w % 32 == 0 && (ci == 16 || ci == 32 || ci == 64 || ci == 96 || ci == 128);
+}
+
+template <int MODE>
+static void launch_conv_lds(const ConvArgs &a, int ci, dim3 grid, hipStream_t st) {
+  switch (ci) {
+    case 16: hipLaunchKernelGGL((k_conv_lds<MODE, 16>), grid, dim3(256), 0, st, a); break;
+    case 32: hipLaunchKernelGGL((k_conv_lds<MODE, 32>), grid, dim3(256), 0, st, a); break;
+    case 64: hipLaunchKernelGGL((k_conv_lds<MODE, 64>), grid, dim3(256), 0, st, a); break;
+    case 96: hipLaunchKernelGGL((k_conv_lds<MODE, 96>), grid, dim3(256), 0, st, a); break;
+    default: hipLaunchKernelGGL((k_conv_lds<MODE, 128>), grid, dim3(256), 0, st, a); break;
+  }
+}
 
 static void launch_conv(int mode, const ConvArgs &a, hipStream_t st) {
   const long long np = (long long)a.nb * a.h * a.wd;
   const int ci = a.ca + a.cs;
   if (conv_lds(np, a.wd, ci)) {
     const dim3 grid((unsigned)(a.nb * ((a.h + 3) / 4) * (a.wd / 32)), (unsigned)(a.co / 32));
-    const size_t lds = conv_lds_bytes(ci);
-    if (mode == 0) hipLaunchKernelGGL(k_conv_lds<0>, grid, dim3(256), lds, st, a);
-    else if (mode == 1) hipLaunchKernelGGL(k_conv_lds<1>, grid, dim3(256), lds, st, a);
-    else hipLaunchKernelGGL(k_conv_lds<2>, grid, dim3(256), lds, st, a);
+    if (mode == 0) launch_conv_lds<0>(a, ci, grid, st);
+    else if (mode == 1) launch_conv_lds<1>(a, ci, grid, st);
+    else launch_conv_lds<2>(a, ci, grid, st);
     return;
   }
   const int ks = conv_ksplit(np, a.co);
