@@ -92,8 +92,8 @@ def load_traffic(name):
 
 
 def run_batch(args):
-    """Config 4: 2048 uneven backward-facing-step channels (D2Q9) advanced in one
-    persistent launch per step, 200-step cycles captured in a hipGraph, each
+    """Config 4: 2048 uneven backward-facing-step channels (D2Q9) advanced by
+    launches over all of them, 200-step cycles captured in a hipGraph, each
     domain retired once its relative residual < 1e-6."""
     import numpy as np
 
