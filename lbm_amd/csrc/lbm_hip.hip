@@ -581,6 +581,7 @@ static int multi3d_fit(const lbm_handle *h) {
 // any.  Without room for it the steps run one per launch.
 static int build_solid3(lbm_handle *h) {
   const int cls = multi3d_fit(h);
+  h->plan3 = Multi3dPlan{};
   if (cls == MULTI3D_NONE) return LBM_OK;
   h->plan3 = multi3d_plan(h->nx, h->ny, h->nz, h->esize, cls);
   if (!h->has_flags) return LBM_OK;
@@ -776,6 +777,7 @@ int lbm_set_bc(lbm_handle *h, const lbm_bc_desc *bcs, int32_t n) {
         return fail(h, LBM_EINVAL, "lbm_set_bc: the faces next to a NEEM wall must be periodic, bounce-back or anti-bounce-back");
     }
   }
+  h->plan3 = Multi3dPlan{};  // until build_links has one for these faces
   memcpy(h->face, face, sizeof(face));
   const int urc = upload_faces(h);
   if (urc) return urc;
@@ -937,7 +939,7 @@ static void launch_multi2d(lbm_handle *h, const Multi2dPlan &p, int cls, int ste
 
 // Plain D3Q19 steps run two per launch (k_multi3d) under the same conditions.
 static int multi3d_cls(const lbm_handle *h) {
-  if (h->w64 || h->lds || !h->wave_paths || (h->has_flags && !h->solid3)) return MULTI3D_NONE;
+  if (!h->plan3.slabs || h->w64 || h->lds || !h->wave_paths || (h->has_flags && !h->solid3)) return MULTI3D_NONE;
   return multi3d_fit(h);
 }
 
