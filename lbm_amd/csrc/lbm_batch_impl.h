@@ -298,9 +298,16 @@ static void domain_tiles(const DomainDev &D, const std::vector<uint8_t> &cc, int
 // Tiles of the multi-step launches (k_multi2d): every active domain cut into
 // equal tiles no larger than the plan's, those without a fluid cell left
 // out.  Empty where the plain steps run one per launch: D3Q19, and batches
-// with a face that kernel has no rule for (multi2d_class).
-static std::vector<MultiTile> multi_tiles(lbm_batch *b) {
-  std::vector<MultiTile> out;
+// with a face that kernel has no rule for (multi2d_class).  The plan belongs
+// to the tiles (its steps fit the LDS on them), so the batch takes all three
+// together.
+struct MultiTiling {
+  std::vector<MultiTile> tiles;
+  Multi2dPlan plan{};
+  int cls = MULTI2D_WALLS;  // the kernel reads every domain's masks
+};
+static MultiTiling multi_tiles(const lbm_batch *b) {
+  MultiTiling out;
   if (b->Q != 9) return out;
   int nx = 0, ny = 0;
   long long cells = 0;
@@ -312,31 +319,30 @@ static std::vector<MultiTile> multi_tiles(lbm_batch *b) {
     cells += (long long)D.nx * D.ny;
   }
   if (!cells) return out;
-  b->mcls = MULTI2D_WALLS;  // the kernel reads every domain's masks
   for (int d = 0; d < b->ndom; ++d) {
     const int cls = multi2d_class(b->doms[d].face, true);
     if (cls == MULTI2D_NONE) return out;
-    b->mcls = std::max(b->mcls, cls);
+    out.cls = std::max(out.cls, cls);
   }
-  b->mplan = multi2d_plan(nx, ny, cells, b->esize, true);
+  out.plan = multi2d_plan(nx, ny, cells, b->esize, true);
   for (int d = 0; d < b->ndom; ++d) {
     if (!b->active_h.empty() && !b->active_h[d]) continue;
     const DomainDev &D = b->doms[d];
     const std::vector<uint8_t> &cc = b->cclass[d];
-    const int cols = (D.nx + b->mplan.tw - 1) / b->mplan.tw, rows = (D.ny + b->mplan.th - 1) / b->mplan.th;
+    const int cols = (D.nx + out.plan.tw - 1) / out.plan.tw, rows = (D.ny + out.plan.th - 1) / out.plan.th;
     // widths in whole groups of 16 cells, so that rows start on the same
     // part of a line
-    const int w = std::min(b->mplan.tw, ((D.nx + cols - 1) / cols + 15) / 16 * 16), h = (D.ny + rows - 1) / rows;
+    const int w = std::min(out.plan.tw, ((D.nx + cols - 1) / cols + 15) / 16 * 16), h = (D.ny + rows - 1) / rows;
     for (int y0 = 0; y0 < D.ny; y0 += h)
       for (int x0 = 0; x0 < D.nx; x0 += w) {
         const MultiTile t{d, x0, y0, std::min(w, D.nx - x0), std::min(h, D.ny - y0)};
         bool fluid = false;
         for (int y = 0; y < t.h && !fluid; ++y)
           for (int x = 0; x < t.w && !fluid; ++x) fluid = cc[(size_t)(x0 + x) + (size_t)D.nx * (y0 + y)] != CELL_SOLID;
-        if (fluid) out.push_back(t);
+        if (fluid) out.tiles.push_back(t);
       }
   }
-  b->mplan.wide = b->mplan.wide && out.size() <= 256;  // one block per CU
+  out.plan.wide = out.plan.wide && out.tiles.size() <= 256;  // one block per CU
   return out;
 }
 
@@ -374,7 +380,8 @@ static int batch_build_tiles(lbm_batch *b, int tx) {
     ids_bnd.push_back(0);
     tiles.push_back(BatchTile{0, 0, 1, 0, 0, 0, 0, 1});  // no lane active
   }
-  std::vector<MultiTile> mtiles = multi_tiles(b);
+  const MultiTiling multi = multi_tiles(b);
+  const std::vector<MultiTile> &mtiles = multi.tiles;
   // launch lists: the interior tiles, the boundary tiles, then every tile in
   // list order (the single-launch form)
   std::vector<int> ids(ids_int);
@@ -408,6 +415,8 @@ static int batch_build_tiles(lbm_batch *b, int tx) {
   if (b->mtiles_d) (void)hipFree(b->mtiles_d);
   b->mtiles_d = mtiles_d;
   b->nmtiles = (int)mtiles.size();
+  b->mplan = multi.plan;
+  b->mcls = multi.cls;
   b->tiles_d = tiles_d;
   b->ids_d = ids_d;
   b->partials = partials;

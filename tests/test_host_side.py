@@ -1,0 +1,88 @@
+"""The host side of liblbm_hip.so on the CPU, over a stand-in for the HIP
+runtime (hip_stand_in.c): which launches a call makes, and what is left of a
+handle when an allocation or a launch fails.  Each test runs in a process of
+its own, where the stand-in takes the runtime's place."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+SETUP = """
+import ctypes as ct, sys
+import numpy as np
+si = ct.CDLL(sys.argv[1], mode=ct.RTLD_GLOBAL)
+from lbm_amd import capi, poisson
+
+def flag(name, kind=ct.c_int):
+    return kind.in_dll(si, name)
+
+class Multi2dArgs(ct.Structure):  # lbm_multi2d.h
+    _fields_ = [("src", ct.c_void_p), ("dst", ct.c_void_p), ("steps", ct.c_int), ("ntiles", ct.c_int),
+                ("plane", ct.c_longlong), ("nx", ct.c_int), ("ny", ct.c_int), ("px", ct.c_int), ("per", ct.c_int * 2),
+                ("face", ct.c_void_p), ("links", ct.c_void_p), ("omega", ct.c_double), ("F", ct.c_double * 3),
+                ("ntx", ct.c_int), ("tw", ct.c_int), ("th", ct.c_int), ("tiles", ct.c_void_p), ("doms", ct.c_void_p),
+                ("active", ct.c_void_p)]
+
+def launches(what, since=0):
+    names = (ct.c_char * 64 * 4096).in_dll(si, "si_name")
+    args = (ct.c_ubyte * 512 * 4096).in_dll(si, "si_args")
+    n = flag("si_launches").value
+    return [(names[k].value.decode(), bytes(args[k])) for k in range(since, min(n, 4096)) if what in names[k].value.decode()]
+
+def count():
+    return flag("si_launches").value
+
+def fail_launch(name, after=0):
+    (ct.c_char * 64).in_dll(si, "si_fail_launch").value = name.encode()
+    flag("si_fail_after").value = after
+
+def multi2d(since=0):
+    return [Multi2dArgs.from_buffer_copy(a) for _, a in launches("k_multi2d", since)]
+"""
+
+
+@pytest.fixture(scope="session")
+def stand_in(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("hip") / "hip_stand_in.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", out, os.path.join(HERE, "hip_stand_in.c")], check=True)
+    return out
+
+
+def run(stand_in, body):
+    env = dict(os.environ, PYTHONPATH=ROOT)
+    r = subprocess.run([sys.executable, "-c", SETUP + body, stand_in], env=env, cwd=ROOT, capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("fails", range(4))  # each allocation of the rebuild
+def test_failed_batch_rebuild_keeps_tiles_and_steps_together(stand_in, fails):
+    """Domains retire, the shorter list of tiles gets another plan (more steps
+    per launch on smaller tiles), and there is no memory for it: the next run
+    goes on with the old tiles, on which the new number of steps does not fit
+    the LDS."""
+    run(stand_in, f"""
+n = 8 * 160 * 128
+b = capi.Batch([{{"shape": (160, 128), "omega": 1.2, "faces": {{}}}}] * 8, storage="f32")
+b.init(np.ones(n), np.zeros((n, 2)))
+def launches_of_a_run():
+    since = count()
+    b.run(50, 0.0, 50)
+    return [(a.steps, a.ntiles, a.tiles) for a in multi2d(since)]
+before = launches_of_a_run()
+flag("si_retire").value = 4
+flag("si_fail_malloc").value = {fails}
+try:
+    b.run(50, 0.0, 50)
+    assert False
+except capi.LBMError as e:
+    assert e.code == capi.LBM_ENOMEM
+flag("si_fail_malloc").value = -1
+assert launches_of_a_run() == before
+b.set_tiling(64, 0)  # succeeds
+assert launches_of_a_run()[0][0] > before[0][0]
+""")

@@ -1,0 +1,36 @@
+"""Calls whose steps go several per launch, in the forms that choose between
+that and one step per launch, against single steps: the populations are equal
+bit for bit."""
+import numpy as np
+import pytest
+
+WALL = ("wall", None, 1.0)
+
+
+def start(shape, seed):
+    rng = np.random.default_rng(seed)
+    n = int(np.prod(shape))
+    return 1 + 1e-3 * rng.standard_normal(n), 0.02 + 2e-3 * rng.standard_normal((n, len(shape)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage", ["f32", "f64"])
+def test_batch_goes_on_after_domains_retire(storage):
+    """Half of the domains are at rest and retire at the first check; the
+    others go on with tiles and steps per launch of the shorter list."""
+    from lbm_amd import capi
+
+    shape, box = (160, 128), {"-x": WALL, "+x": WALL, "-y": WALL, "+y": WALL}
+    fields = [start(shape, k) if k % 2 else (np.ones(160 * 128), np.zeros((160 * 128, 2))) for k in range(8)]
+    b = capi.Batch([{"shape": shape, "omega": 1.0 + 0.05 * k, "faces": box} for k in range(8)], storage=storage)
+    b.init(np.concatenate([f[0] for f in fields]), np.concatenate([f[1] for f in fields]))
+    steps = b.run(26, 1e-300, 78)[0]
+    assert [int(s) for s in steps] == [-1 if k % 2 else 26 for k in range(8)]
+    for k in range(8):
+        lat = capi.Lattice(shape, storage=storage, omega=1.0 + 0.05 * k, faces=box)
+        lat.init(*fields[k])
+        for _ in range(78 if k % 2 else 26):
+            lat.step(1)
+        assert np.array_equal(b.populations(k), lat.populations()), k
+        lat.close()
+    b.close()
