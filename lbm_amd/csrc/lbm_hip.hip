@@ -546,7 +546,7 @@ __global__ void __launch_bounds__(256) k_lanes(const uint32_t *links, int nx, in
   if ((t & 63) == 0) lanes[wave] = m;
 }
 
-static Multi3dArgs multi3d_args(const lbm_handle *h) {
+static Multi3dArgs multi3d_args(const lbm_handle *h, const Multi3dPlan &p) {
   Multi3dArgs a;
   memset(&a, 0, sizeof(a));
   a.plane = h->plane;
@@ -560,7 +560,6 @@ static Multi3dArgs multi3d_args(const lbm_handle *h) {
   a.solid = h->solid3;
   a.omega = h->omega;
   for (int i = 0; i < 3; ++i) a.F[i] = h->F[i];
-  const Multi3dPlan &p = h->plan3;
   a.tw = p.tw;
   a.ntx = p.ntx;
   a.nty = p.nty;
@@ -578,28 +577,30 @@ static int multi3d_fit(const lbm_handle *h) {
 
 // The two-step kernel's tiles, and its blocks that meet a solid.  Their number
 // depends on the storage form (the tile does), so the array holds the most of
-// any.  Without room for it the steps run one per launch.
-static int build_solid3(lbm_handle *h) {
+// any.  The handle takes the plan last: without room for the array, or where
+// the launch that fills it fails, it has none and the steps run one per launch.
+static void build_solid3(lbm_handle *h) {
   const int cls = multi3d_fit(h);
   h->plan3 = Multi3dPlan{};
-  if (cls == MULTI3D_NONE) return LBM_OK;
-  h->plan3 = multi3d_plan(h->nx, h->ny, h->nz, h->esize, cls);
-  if (!h->has_flags) return LBM_OK;
-  if (!h->solid3) {
-    long long n = 0;
-    for (int es : {4, 8}) {
-      const Multi3dPlan p = multi3d_plan(h->nx, h->ny, h->nz, es, MULTI3D_WALLS);
-      n = std::max(n, (long long)p.ntx * p.nty * p.slabs);
+  if (cls == MULTI3D_NONE) return;
+  const Multi3dPlan plan = multi3d_plan(h->nx, h->ny, h->nz, h->esize, cls);
+  if (h->has_flags) {
+    if (!h->solid3) {
+      long long n = 0;
+      for (int es : {4, 8}) {
+        const Multi3dPlan p = multi3d_plan(h->nx, h->ny, h->nz, es, MULTI3D_WALLS);
+        n = std::max(n, (long long)p.ntx * p.nty * p.slabs);
+      }
+      if (hipMalloc(&h->solid3, (size_t)n) != hipSuccess) {
+        (void)hipGetLastError();
+        h->solid3 = nullptr;
+        return;
+      }
     }
-    if (hipMalloc(&h->solid3, (size_t)n) != hipSuccess) {
-      (void)hipGetLastError();
-      h->solid3 = nullptr;
-      return LBM_OK;
-    }
+    multi3d_solid(multi3d_args(h, plan), h->solid3, h->stream);
+    if (hipGetLastError() != hipSuccess) return;
   }
-  multi3d_solid(multi3d_args(h), h->solid3, h->stream);
-  HIPCHK(h, hipGetLastError());
-  return LBM_OK;
+  h->plan3 = plan;
 }
 
 // (Re)build the solid-link masks and the interior lanes; they depend on the
@@ -617,7 +618,8 @@ static int build_links(lbm_handle *h) {
                        h->nz, h->px, h->dim, h->lanes);
     HIPCHK(h, hipGetLastError());
   }
-  return build_solid3(h);
+  build_solid3(h);
+  return LBM_OK;
 }
 
 extern "C" {
@@ -939,7 +941,7 @@ static void launch_multi2d(lbm_handle *h, const Multi2dPlan &p, int cls, int ste
 
 // Plain D3Q19 steps run two per launch (k_multi3d) under the same conditions.
 static int multi3d_cls(const lbm_handle *h) {
-  if (!h->plan3.slabs || h->w64 || h->lds || !h->wave_paths || (h->has_flags && !h->solid3)) return MULTI3D_NONE;
+  if (!h->plan3.slabs || h->w64 || h->lds || !h->wave_paths) return MULTI3D_NONE;
   return multi3d_fit(h);
 }
 
@@ -957,7 +959,7 @@ int lbm_step(lbm_handle *h, int32_t nsteps) {
   }
   const int cls3 = multi3d_cls(h);
   if (nsteps > 1 && cls3 != MULTI3D_NONE) {
-    Multi3dArgs a = multi3d_args(h);
+    Multi3dArgs a = multi3d_args(h, h->plan3);
     for (; nsteps > 1; nsteps -= 2) {
       a.src = h->buf[h->cur];
       a.dst = h->buf[h->cur ^ 1];
@@ -1146,7 +1148,8 @@ int lbm_set_storage(lbm_handle *h, int32_t storage) {
   h->w64 = (unsigned long long)h->plane * (unsigned long long)es > 0xffffffffull;
   h->snap_last = 0;
   if (storage != LBM_STORE_F32) h->lds = false;
-  return build_solid3(h);
+  build_solid3(h);
+  return LBM_OK;
 }
 
 int lbm_time_steps(lbm_handle *h, int32_t nsteps, double *ms) {

@@ -86,3 +86,33 @@ assert launches_of_a_run() == before
 b.set_tiling(64, 0)  # succeeds
 assert launches_of_a_run()[0][0] > before[0][0]
 """)
+
+
+@pytest.mark.parametrize("call", ["set_storage", "set_faces"])
+def test_without_block_flags_steps_run_one_per_launch(stand_in, call):
+    """The launch that marks the two-step kernel's blocks that meet a solid
+    fails: the call succeeds, the marks of the old storage form's tiles (or
+    none) are not used with the new tiles, and a later call makes them."""
+    run(stand_in, f"""
+wall = ("wall", None, 1.0)
+faces = {{"-y": wall, "+y": wall, "-z": wall, "+z": wall}}
+solid = np.zeros((64, 100, 128), np.uint8)
+solid[20:30, 20:30, 20:30] = 1
+lat = capi.Lattice((128, 100, 64), storage="f64", omega=1.2, faces=faces, solid=solid)
+def kernels_of_two_steps():
+    since = count()
+    lat.step(2)
+    return [n for n, _ in launches("", since)]
+assert len(launches("k_multi3d_solid")) == 2 and ["k_multi3d" in n for n in kernels_of_two_steps()] == [True]
+def change(k):
+    if "{call}" == "set_storage":
+        lat.set_storage("f32" if k else "f64")
+    else:
+        lat.set_faces(dict(faces, **{{"+z": ("wall", (0.01 * k, 0.0, 0.0), 1.0)}}))
+fail_launch("k_multi3d_solid")
+change(1)
+assert ["k_multi3d" in n for n in kernels_of_two_steps()] == [False, False]
+fail_launch("")
+change(0)
+assert ["k_multi3d" in n for n in kernels_of_two_steps()] == [True]
+""")
