@@ -74,7 +74,8 @@ int lbm_batch_init_fields(lbm_batch *b, const double *rho, const double *u);
 int lbm_batch_run(lbm_batch *b, int32_t interval, double tol, int64_t max_steps, lbm_domain_result *results,
                   double *ms);
 
-/* Macroscopic fields of one domain (compact layout). */
+/* Macroscopic fields of one domain (compact layout).  Reads of a batch's
+ * domains may come from several host threads; they go in turn. */
 int lbm_batch_get_macros(lbm_batch *b, int32_t dom, double *rho, double *u);
 
 /* Post-collision populations of one domain, SoA [Q][cells], FP64. */

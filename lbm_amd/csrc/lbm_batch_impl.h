@@ -843,6 +843,7 @@ int lbm_batch_run(lbm_batch *b, int32_t interval, double tol, int64_t max_steps,
 
 int lbm_batch_get_macros(lbm_batch *b, int32_t dom, double *rho, double *u) {
   if (!b || dom < 0 || dom >= b->ndom || !rho || !u) return bfail(b, LBM_EINVAL, "lbm_batch_get_macros: bad argument");
+  const auto staging = b->out.hold();
   const DomainDev &D = b->doms[dom];
   const long long n = (long long)D.nx * D.ny * D.nz;
   const size_t bytes = (size_t)n * (1 + b->dim) * sizeof(double);
@@ -879,6 +880,7 @@ int lbm_batch_get_macros(lbm_batch *b, int32_t dom, double *rho, double *u) {
 
 int lbm_batch_get_populations(lbm_batch *b, int32_t dom, double *f) {
   if (!b || dom < 0 || dom >= b->ndom || !f) return bfail(b, LBM_EINVAL, "lbm_batch_get_populations: bad argument");
+  const auto staging = b->out.hold();
   const DomainDev &D = b->doms[dom];
   const long long n = (long long)D.nx * D.ny * D.nz;
   DevBuf fbuf;

@@ -1042,6 +1042,7 @@ int lbm_step_ex_noalloc(lbm_handle *h, int32_t mode, lbm_sums *out) {
 
 int lbm_get_macros(lbm_handle *h, double *rho, double *u) {
   if (!h || !rho || !u) return fail(h, LBM_EINVAL, "lbm_get_macros: null argument");
+  const auto staging = h->out.hold();
   const int rc = ensure_io(h, (size_t)h->ncell * (1 + h->dim) * sizeof(double));
   if (rc) return rc;
   double *rd = static_cast<double *>(h->io), *ud = rd + h->ncell;
@@ -1082,6 +1083,7 @@ int lbm_reduce(lbm_handle *h, lbm_sums *out) {
 
 int lbm_get_populations(lbm_handle *h, double *f) {
   if (!h || !f) return fail(h, LBM_EINVAL, "lbm_get_populations: null argument");
+  const auto staging = h->out.hold();
   const size_t bytes = (size_t)h->ncell * h->Q * sizeof(double);
   DevBuf fd;
   HIPCHK(h, fd.alloc(bytes));

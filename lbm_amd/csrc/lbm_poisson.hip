@@ -686,6 +686,7 @@ int lbm_poisson_step_check(lbm_poisson *h, double *abs_diff) {
 
 int lbm_poisson_get(lbm_poisson *h, double *phi) {
   if (!h || !phi) return pfail(h, LBM_EINVAL, "lbm_poisson_get: null argument");
+  const auto staging = h->out.hold();
   hipLaunchKernelGGL(k_poisson_compact, pgrid(h), dim3(256), 0, h->stream, (const double *)h->phi[h->pcur], h->nx, h->ny,
                      h->px, h->io);
   PCHK(h, hipGetLastError());

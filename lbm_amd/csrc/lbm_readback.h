@@ -19,10 +19,14 @@ namespace lbm {
 // MB 51 -> 14 ms, 50 MB 4.0 -> 1.8 ms, once 2 ms more for the chunks; 8 MB 0.5
 // ms either way, so smaller copies stay with the runtime).  The chunks stay
 // with the owner; threads live as long as the call.
+// A read-back holds the staging (hold()) from the kernel that fills it to the
+// end of its copy: reads of one owner from several threads go in turn.
 class Readback {
  public:
   static constexpr size_t CHUNK = 2u << 20;
   static constexpr int THREADS = 8, CHUNKS = 2 * THREADS;
+
+  std::unique_lock<std::mutex> hold() { return std::unique_lock<std::mutex>(mu_); }
 
   // two arrays that lie one behind the other at src
   hipError_t copy(void *dst, size_t bytes, void *dst2, size_t bytes2, const void *src, hipStream_t s) {
@@ -140,6 +144,7 @@ class Readback {
     }
     return true;
   }
+  std::mutex mu_;
   void *chunk_[CHUNKS] = {};
   hipEvent_t event_[CHUNKS] = {};
   int have_ = 0;
