@@ -749,7 +749,7 @@ static int batch_plain(lbm_batch *b, int parity, int steps) {
     for (int s = 0; s < steps; ++s) batch_launch(b, (parity + s) & 1, 0);
     return (parity + steps) & 1;
   }
-  int n = (steps + b->mplan.steps - 1) / b->mplan.steps;
+  int n = steps / b->mplan.steps + (steps % b->mplan.steps != 0);
   n += (n ^ steps) & 1;  // the parity that single steps end with
   for (int i = 0; i < n; ++i) {
     Multi2dArgs a;

@@ -950,7 +950,7 @@ int lbm_step(lbm_handle *h, int32_t nsteps) {
   const int cls = multi2d_cls(h);
   if (nsteps > 1 && cls != MULTI2D_NONE) {
     const Multi2dPlan p = multi2d_plan(h->nx, h->ny, h->ncell, h->esize, cls != MULTI2D_BOX);
-    const int n = (nsteps + p.steps - 1) / p.steps;
+    const int n = nsteps / p.steps + (nsteps % p.steps != 0);
     for (int i = 0; i < n; ++i) {  // as even as possible
       launch_multi2d(h, p, cls, nsteps / n + (i < nsteps % n ? 1 : 0));
       HIPCHK(h, hipGetLastError());

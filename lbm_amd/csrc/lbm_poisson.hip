@@ -541,9 +541,9 @@ static PMulti multi_plan(const lbm_poisson *h) {
 // nsteps > 1 plain steps, split evenly over the launches.  The last two
 // states of phi go to the two slots that the next step reads and the one
 // after it.
-static void launch_multi(lbm_poisson *h, int nsteps) {
+static int launch_multi(lbm_poisson *h, int nsteps) {
   PMulti m = multi_plan(h);
-  const int n = (nsteps + m.steps - 1) / m.steps;
+  const int n = nsteps / m.steps + (nsteps % m.steps != 0);
   bool neumann = false;
   for (int f = 0; f < 4; ++f) neumann = neumann || h->kind[f] == LBM_POISSON_NEUMANN;
   const dim3 g((m.ntiles + 7) / 8 * 8), b(MULTI_THREADS);
@@ -557,9 +557,11 @@ static void launch_multi(lbm_poisson *h, int nsteps) {
     if (h->Q == 3) hipLaunchKernelGGL(k_poisson_multi<3>, g, b, 0, h->stream, a, m);
     else if (h->Q == 5) hipLaunchKernelGGL(k_poisson_multi<5>, g, b, 0, h->stream, a, m);
     else hipLaunchKernelGGL(k_poisson_multi<9>, g, b, 0, h->stream, a, m);
+    PCHK(h, hipGetLastError());
     h->cur ^= 1;
     h->pcur = (h->pcur + 2) % 3;
   }
+  return LBM_OK;
 }
 
 extern "C" {
@@ -664,8 +666,8 @@ int lbm_poisson_init(lbm_poisson *h, const double *phi0) {
 int lbm_poisson_step(lbm_poisson *h, int32_t nsteps) {
   if (!h || nsteps < 0) return pfail(h, LBM_EINVAL, "lbm_poisson_step: bad argument");
   if (!h->ready) return pfail(h, LBM_EINVAL, "lbm_poisson_step: lbm_poisson_init first");
+  if (nsteps > 1) return launch_multi(h, nsteps);
   if (nsteps == 1) launch_step<false>(h);
-  if (nsteps > 1) launch_multi(h, nsteps);
   PCHK(h, hipGetLastError());
   return LBM_OK;
 }

@@ -116,3 +116,26 @@ fail_launch("")
 change(0)
 assert ["k_multi3d" in n for n in kernels_of_two_steps()] == [True]
 """)
+
+
+def test_as_many_steps_as_the_argument_holds(stand_in):
+    """2^31 - 1 steps are launched (until the stand-in lets a launch fail)."""
+    run(stand_in, """
+def fails_on_the_way(step, kernel):
+    since = count()
+    fail_launch(kernel, after=5)
+    try:
+        step(2 ** 31 - 1)
+        assert False
+    except RuntimeError:
+        pass
+    fail_launch("")
+    assert len(launches(kernel, since)) == 5
+lat = capi.Lattice((64, 32), omega=1.2)
+fails_on_the_way(lat.step, "k_multi2d")
+assert multi2d()[0].steps == 8
+p = poisson.Poisson(5, 64, 32, 1.0, 0.0)
+p.set_faces({f: ("neumann", None, k) for k, f in enumerate(("-x", "+x", "-y", "+y"))})
+p.init(np.zeros(64 * 32))
+fails_on_the_way(p.step, "k_poisson_multi")
+""")
