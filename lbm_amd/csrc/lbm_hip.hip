@@ -914,7 +914,7 @@ static int multi2d_cls(const lbm_handle *h) {
   return multi2d_class(h->face, h->has_flags);
 }
 
-static void launch_multi2d(lbm_handle *h, const Multi2dPlan &p, int cls, int steps) {
+static int launch_multi2d(lbm_handle *h, const Multi2dPlan &p, int cls, int steps) {
   Multi2dArgs a;
   memset(&a, 0, sizeof(a));
   a.src = h->buf[h->cur];
@@ -935,8 +935,10 @@ static void launch_multi2d(lbm_handle *h, const Multi2dPlan &p, int cls, int ste
   a.th = p.th;
   a.ntiles = a.ntx * ((h->ny + p.th - 1) / p.th);
   dispatch_s<Multi2dL>(h->storage, a, h->stream, cls, p.wide);
+  HIPCHK(h, hipGetLastError());
   h->cur ^= 1;
   h->steps += steps;
+  return LBM_OK;
 }
 
 // Plain D3Q19 steps run two per launch (k_multi3d) under the same conditions.
@@ -952,8 +954,8 @@ int lbm_step(lbm_handle *h, int32_t nsteps) {
     const Multi2dPlan p = multi2d_plan(h->nx, h->ny, h->ncell, h->esize, cls != MULTI2D_BOX);
     const int n = nsteps / p.steps + (nsteps % p.steps != 0);
     for (int i = 0; i < n; ++i) {  // as even as possible
-      launch_multi2d(h, p, cls, nsteps / n + (i < nsteps % n ? 1 : 0));
-      HIPCHK(h, hipGetLastError());
+      const int rc = launch_multi2d(h, p, cls, nsteps / n + (i < nsteps % n ? 1 : 0));
+      if (rc) return rc;
     }
     return LBM_OK;
   }

@@ -139,3 +139,21 @@ p.set_faces({f: ("neumann", None, k) for k, f in enumerate(("-x", "+x", "-y", "+
 p.init(np.zeros(64 * 32))
 fails_on_the_way(p.step, "k_poisson_multi")
 """)
+
+
+def test_a_failed_launch_leaves_the_state_current(stand_in):
+    """The next launch reads the state that the failed one would have read."""
+    run(stand_in, """
+lat = capi.Lattice((64, 32), omega=1.2)
+lat.step(8)
+fail_launch("k_multi2d")
+try:
+    lat.step(8)
+    assert False
+except capi.LBMError as e:
+    assert e.code == capi.LBM_EHIP
+fail_launch("")
+lat.step(8)
+first, after = multi2d()
+assert after.src == first.dst and after.dst == first.src
+""")
