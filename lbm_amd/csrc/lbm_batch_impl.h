@@ -310,12 +310,15 @@ static MultiTiling multi_tiles(const lbm_batch *b) {
   MultiTiling out;
   if (b->Q != 9) return out;
   int nx = 0, ny = 0;
+  bool pery = false, solids = false;
   long long cells = 0;
   for (int d = 0; d < b->ndom; ++d) {
     const DomainDev &D = b->doms[d];
     if (!b->active_h.empty() && !b->active_h[d]) continue;
     nx = std::max(nx, D.nx);
     ny = std::max(ny, D.ny);
+    pery = pery || D.per[1];
+    solids = solids || !b->solid[d].empty();
     cells += (long long)D.nx * D.ny;
   }
   if (!cells) return out;
@@ -324,7 +327,8 @@ static MultiTiling multi_tiles(const lbm_batch *b) {
     if (cls == MULTI2D_NONE) return out;
     out.cls = std::max(out.cls, cls);
   }
-  out.plan = multi2d_plan(nx, ny, cells, b->esize, true);
+  out.plan = multi2d_plan({nx, ny, cells, b->esize, true, pery, solids, FORCE_NONE});
+  if (out.plan.steps < 2) return out;
   for (int d = 0; d < b->ndom; ++d) {
     if (!b->active_h.empty() && !b->active_h[d]) continue;
     const DomainDev &D = b->doms[d];

@@ -907,8 +907,9 @@ static int finalize_sums(lbm_handle *h, lbm_sums *out) {
 
 // Plain D2Q9 steps run several per launch (k_multi2d) unless a face needs
 // more than that kernel has (multi2d_class), the forcing correction runs
-// between steps, a plane needs 64-bit offsets, or the handle was set to the
-// general path of the single-step kernel or to its LDS halo.
+// between steps, a plane needs 64-bit offsets, the handle was set to the
+// general path of the single-step kernel or to its LDS halo, or the domain
+// has so few rows that one step per launch is faster (multi2d_plan).
 static int multi2d_cls(const lbm_handle *h) {
   if (h->Q != 9 || h->forcing || h->w64 || h->lds || !h->wave_paths) return MULTI2D_NONE;
   return multi2d_class(h->face, h->has_flags);
@@ -949,9 +950,11 @@ static int multi3d_cls(const lbm_handle *h) {
 
 int lbm_step(lbm_handle *h, int32_t nsteps) {
   if (!h || nsteps < 0) return fail(h, LBM_EINVAL, "lbm_step: bad argument");
-  const int cls = multi2d_cls(h);
-  if (nsteps > 1 && cls != MULTI2D_NONE) {
-    const Multi2dPlan p = multi2d_plan(h->nx, h->ny, h->ncell, h->esize, cls != MULTI2D_BOX);
+  const int cls = nsteps > 1 ? multi2d_cls(h) : MULTI2D_NONE;
+  Multi2dPlan p{1, 0, 0, false};
+  if (cls != MULTI2D_NONE)
+    p = multi2d_plan({h->nx, h->ny, h->ncell, h->esize, cls != MULTI2D_BOX, h->per[1] != 0, h->has_flags, force_kind(h->F)});
+  if (p.steps > 1) {
     const int n = nsteps / p.steps + (nsteps % p.steps != 0);
     for (int i = 0; i < n; ++i) {  // as even as possible
       const int rc = launch_multi2d(h, p, cls, nsteps / n + (i < nsteps % n ? 1 : 0));

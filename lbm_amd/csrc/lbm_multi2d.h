@@ -84,13 +84,30 @@ __host__ __device__ inline int multi2d_slots(int w, int h, int steps) {
   return (w + 2 * steps) * (h + 2 * steps) + 4 * steps;
 }
 
-// Steps per launch and tile of a domain of nx x ny cells, `cells` in the
-// whole launch.
+// Whether the kernel's row of a linear index is exact for a tile of `slots`
+// slots in lines of `pitch`: i * (2^20 / w + 1) is above 2^20 i / w by at most
+// i, less than the 2^20 / w to the next row.  The general plan's lines are at
+// most 144 long (128 cells and 8 steps) and every tile fits multi2d_cap.
+constexpr bool multi2d_exact(int slots, int pitch) { return (long long)slots * pitch < 1 << 20; }
+static_assert(multi2d_exact(multi2d_cap(2, false), 144), "the widest tiles of the general plan");
+
+// What a plan depends on: a domain of nx x ny cells, `cells` in the whole
+// launch.
+struct Multi2dDomain {
+  int nx, ny;
+  long long cells;
+  int esize;
+  bool faces;   // not MULTI2D_BOX
+  bool pery;    // the y axis is periodic
+  bool solids;
+  int force;    // force_kind
+};
+// Steps per launch and tile.  steps 1: the single-step kernels are faster.
 struct Multi2dPlan {
   int steps, tw, th;
   bool wide;
 };
-Multi2dPlan multi2d_plan(int nx, int ny, long long cells, int esize, bool faces);
+Multi2dPlan multi2d_plan(const Multi2dDomain &d);
 
 template <typename ST>
 struct Multi2dL {

@@ -206,7 +206,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
   auto faces_of = [&](int x, int y) {
     return (x == flo0 ? 1u : 0u) | (x == fhi0 ? 2u : 0u) | (y == flo1 ? 4u : 0u) | (y == fhi1 ? 8u : 0u);
   };
-  // row of a linear index: exact for indices below 2^13 and widths below 2^7
+  // row of a linear index: exact where index * width < 2^20 (multi2d_exact)
   auto recip = [](int w) { return (unsigned)((1 << 20) / w + 1); };
   {
     const unsigned rp = recip(pitch);
@@ -289,6 +289,36 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
   }
 }
 
+// Microseconds per step of a plan, and of one step per launch, fitted to 1300
+// timings of domains of 3 to 40 rows (5 % in the mean for tiles of the least
+// time, up to 25 % for FP64 and for tiles with idle threads).  A tile's work
+// counts whole waves and a fixed part per step, more where cells have masks;
+// `rounds` as in general_plan.
+static double multi2d_time(const Multi2dDomain &d, const Multi2dPlan &p) {
+  constexpr int NCU = 256;
+  const int tw = p.tw, th = p.th, t = p.steps, whole = d.faces ? 256 : 128;
+  auto at = [&](int back) { return (long long)(tw + 2 * back) * (d.pery ? th + 2 * back : std::min(th + 2 * back, d.ny)); };
+  auto full = [&](long long n) { return (double)((n + whole - 1) / whole * whole); };
+  double work = full(at(t));
+  for (int s = 0; s < t; ++s) work += full(at(s)) + (d.faces ? 350.0 : 250.0);
+  const long long columns = (d.cells + (long long)tw * d.ny - 1) / ((long long)tw * d.ny),
+                  tiles = columns * ((d.ny + th - 1) / th), rest = tiles % (2 * NCU);
+  const double rounds = 2.0 * (double)(tiles / (2 * NCU)) + (rest == 0 ? 0.0 : rest <= NCU ? 1.3 : 2.0);
+  const double unit = (d.esize == 4 ? 1.02e-3 : d.esize == 8 ? 0.95e-3 : 0.85e-3) * (d.faces ? 1.14 : 1.0) *
+                      (1.0 + d.force * (d.esize == 4 ? 0.12 : d.esize == 8 ? 0.06 : 0.1));
+  const double us = unit * (rounds * work + 3000.0) / t;
+  // beyond the cache: 4.8 TB/s
+  const double moved = (double)d.cells * 9 * d.esize * (1.0 + (double)at(t) / (tw * th)) / t / 4.8e6;
+  return 2 * 9 * d.esize * d.cells > (256ll << 20) ? std::max(us, moved) : us;
+}
+static double single2d_time(const Multi2dDomain &d) {
+  const int bx = d.nx > 128 ? 256 : d.nx > 64 ? 128 : 64;
+  // lanes, at the rate of cells without solids; 10 % of solids take 1.67 times
+  const double lanes = (double)((d.nx + bx - 1) / bx * bx) * (double)(d.cells / d.nx) * (d.solids ? 1.35 : 1.0);
+  if (d.esize == 2) return d.faces ? 3.9 + 8.8e-6 * lanes : 2.6 + 6.6e-6 * lanes;
+  return (d.faces ? 3.5 : 2.8) + (d.esize == 4 ? 12.8e-6 : 24.5e-6) * lanes;
+}
+
 // Tiles of a power of two of cells, as square as it gets: about one per CU as
 // long as that leaves at least 64 cells and at most 4 KB per direction (512,
 // 1024 or 2048 cells), which with the halo is what two blocks of a CU hold.
@@ -310,9 +340,12 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 //   4096 x 2048 FP32  64 x 20, 4      68       32 x 32, 6   70      119
 //   2048^2 FP64       32 x 16, 4      51       32 x 20, 3   58      113
 //   4096 x 2048 FP16  128 x 20, 4     56       64 x 32, 6   56       81
-Multi2dPlan multi2d_plan(int nx, int ny, long long cells, int esize, bool faces) {
+static Multi2dPlan general_plan(const Multi2dDomain &d) {
   constexpr int NCU = 256;
   constexpr long long CACHE = 256ll << 20;
+  const int nx = d.nx, ny = d.ny, esize = d.esize;
+  const long long cells = d.cells;
+  const bool faces = d.faces;
   const int cap = multi2d_cap(esize, faces), most = 4096 / esize;
   Multi2dPlan p;
   if (2 * 9 * esize * cells > CACHE) {
@@ -345,6 +378,40 @@ Multi2dPlan multi2d_plan(int nx, int ny, long long cells, int esize, bool faces)
     p.wide = tiles <= NCU && p.tw * th >= 256;
   }
   return p;
+}
+
+// Domains of few rows: a tile of the rule above holds too few cells for its
+// threads there, and the rows of a periodic axis are updated several times
+// over (3 rows and 6 steps: 3 times).  Wider tiles with fewer steps, or one
+// step per launch where even these take longer, by multi2d_time (below 2^15
+// cells the launch is all there is to save, and the rule above holds).
+// Microseconds per step, one step per launch, the rule above, this one:
+//   333333 x 3 FP32 periodic   15.5   30.6   14.2 (256 x 3, 2 steps)
+//   333333 x 3 FP16 periodic    8.9   18.1    8.8 (one step per launch)
+//   1333333 x 3 FP16 walls     46     63     33   (256 x 3, 4 steps)
+//   250000 x 4 FP32 NEEM       16.7   29.6   14.1 (128 x 4, 4 steps)
+//   100000 x 10 FP32 periodic  15.5   13.8   12.0
+// From 32 rows on the rule above is never slower than 1.05 times one step per
+// launch (25000 x 40 FP16, periodic with a force along y: 9.8 against 9.3).
+Multi2dPlan multi2d_plan(const Multi2dDomain &d) {
+  constexpr int THIN = 32;
+  const Multi2dPlan general = general_plan(d);
+  if (d.ny >= THIN || d.cells < 1 << 15) return general;
+  Multi2dPlan best = general;
+  const int cap = multi2d_cap(d.esize, d.faces);
+  double time = multi2d_time(d, general), least = 0.8 * time;  // the fit has to be sure
+  for (int rows = 1; rows <= 3; ++rows)
+    for (int width = 32; width <= 512; width *= 2)
+      for (int t : {2, 3, 4, 6, 8}) {
+        const Multi2dPlan p{t, std::min(width, d.nx), (d.ny + rows - 1) / rows, false};
+        const int slots = multi2d_slots(p.tw, p.th, t);
+        if (slots > cap || !multi2d_exact(slots, p.tw + 2 * t)) continue;
+        const double us = multi2d_time(d, p);
+        if (us >= least) continue;
+        time = least = us;
+        best = p;
+      }
+  return time > single2d_time(d) ? Multi2dPlan{1, 0, 0, false} : best;
 }
 
 template <typename ST, int FORCE, int NT>

@@ -157,3 +157,73 @@ lat.step(8)
 first, after = multi2d()
 assert after.src == first.dst and after.dst == first.src
 """)
+
+
+TILES = """
+def extent(b, e, back, n, periodic):
+    if periodic:
+        return b - back, e + back
+    if back:
+        b, e = min(b, n - 2), max(e, 1)
+    return max(b - back, 0), min(e + back, n - 1)
+
+def slots(x0, x1, y0, y1, nx, ny, T, perx, pery, open_faces):
+    '''LDS slots per direction of a tile (k_multi2d): its region and what the
+    in-place steps, each a line or two further down, need in front'''
+    rx, ry = extent(x0, x1, T, nx, perx), extent(y0, y1, T, ny, pery)
+    pitch, rows = rx[1] - rx[0] + 1, ry[1] - ry[0] + 1
+    columns = not perx and (rx[0] == 0 and open_faces or rx[1] == nx - 1 and open_faces)
+    sx, sy = (rows, 1) if columns else (1, pitch)
+    pad = down = 0
+    for s in range(1, T):
+        ex, ey = extent(x0, x1, T - s, nx, perx), extent(y0, y1, T - s, ny, pery)
+        down += ((2 if ex[1] == nx - 1 else 1) * rows if columns else pitch) + 2
+        pad = max(pad, down - (ey[0] - ry[0]) * sy - (ex[0] - rx[0]) * sx)
+    assert pitch * rows * max(pitch, rows) < 1 << 20  # the kernel's division by a line
+    return pad + pitch * rows
+
+def updates(a, pery):
+    '''cells updated per cell kept and step'''
+    return sum((a.tw + 2 * s) * (a.th + 2 * s if pery else min(a.th + 2 * s, a.ny)) for s in range(a.steps)) / \\
+        (a.steps * a.tw * min(a.th, a.ny))
+"""
+
+
+@pytest.mark.parametrize("storage,esize", [("f32", 4), ("f64", 8), ("f16", 2)])
+@pytest.mark.parametrize("faces", ["periodic", "walls", "neem"])
+def test_low_domains(stand_in, storage, esize, faces):
+    """Domains of few rows: every tile fits the LDS, rows of a periodic axis are
+    not updated several times over, and where tiles of so few rows take longer
+    than one step per launch there are none."""
+    run(stand_in, TILES + f"""
+wall = ("wall", None, 1.0)
+kinds = {{"periodic": {{}}, "walls": {{"-y": wall, "+y": wall}},
+         "neem": {{"-y": wall, "+y": wall, "-x": ("velocity_neem", (0.01, 0.0), 1.0), "+x": ("pressure_neem", None, 1.0)}}}}
+box = "{faces}" == "periodic"
+cap = (80 * 1024 - 256) // (9 * {esize} + (0 if box else 2)) // 16 * 16
+for ny in list(range(3, 34)) + [48, 63]:
+    for cells in (100, 3000, 30000, 400000, 1500000):
+        nx = max(3, cells // ny)
+        lat = capi.Lattice((nx, ny), storage="{storage}", omega=1.2, faces=kinds["{faces}"])
+        since = count()
+        lat.step(24)
+        lat.close()
+        plans = multi2d(since)
+        assert plans or (ny < 32 and cells >= 30000), (nx, ny)
+        if not plans:
+            assert len(launches("k_step", since)) == 24
+            continue
+        a = plans[0]
+        if cells >= 400000 and ny < 32:
+            assert updates(a, box) < 2.0, (nx, ny, a.tw, a.th, a.steps)
+        edge = lambda n, w: sorted({{0, w, n // w // 2 * w, (n - 1) // w * w - w, (n - 1) // w * w}} & set(range(0, n, w)))
+        for x0 in edge(nx, a.tw):
+            for y0 in edge(ny, a.th):
+                n = slots(x0, min(x0 + a.tw, nx) - 1, y0, min(y0 + a.th, ny) - 1, nx, ny, a.steps, "{faces}" != "neem", box,
+                          "{faces}" == "neem")
+                assert n <= cap, (nx, ny, a.tw, a.th, a.steps, x0, y0, n)
+lat = capi.Lattice((1 << 20, 3), storage="f16", omega=1.2)
+since = count()
+lat.step(24)
+assert len(launches("k_step", since)) == 24
+""")

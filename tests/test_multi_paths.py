@@ -34,3 +34,26 @@ def test_batch_goes_on_after_domains_retire(storage):
         assert np.array_equal(b.populations(k), lat.populations()), k
         lat.close()
     b.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage", ["f32", "f64", "f16"])
+@pytest.mark.parametrize("faces", ["periodic", "walls", "neem"])
+def test_low_domains_equal_single_steps(storage, faces):
+    """Few rows: wide tiles, two to eight steps per launch, or one."""
+    from lbm_amd import capi
+
+    walls = {"-y": WALL, "+y": ("wall", (0.02, 0.0), 1.0)}
+    kinds = {"periodic": {}, "walls": walls,
+             "neem": dict(walls, **{"-x": ("velocity_neem", (0.03, 0.0), 1.0), "+x": ("pressure_neem", None, 1.0)})}
+    for nx, ny in ((701, 3), (40000, 3), (300000, 3), (30011, 5), (250007, 6), (33, 12), (20001, 17), (60000, 31)):
+        solid = (np.random.default_rng(ny).random(nx * ny) < 0.05).astype(np.uint8) if ny > 5 else None
+        out = []
+        for calls in ((17, 2, 5), (1,) * 24):
+            lat = capi.Lattice((nx, ny), storage=storage, omega=1.2, faces=kinds[faces], solid=solid)
+            lat.init(*start((nx, ny), ny))
+            for n in calls:
+                lat.step(n)
+            out.append(lat.populations())
+            lat.close()
+        assert np.isfinite(out[0]).all() and np.array_equal(*out), (nx, ny)
