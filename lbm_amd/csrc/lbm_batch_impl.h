@@ -311,7 +311,7 @@ static MultiTiling multi_tiles(const lbm_batch *b) {
   if (b->Q != 9) return out;
   int nx = 0, ny = 0;
   bool pery = false, solids = false;
-  long long cells = 0;
+  long long cells = 0, low = 0;  // low: of few rows that are updated again for the halo
   for (int d = 0; d < b->ndom; ++d) {
     const DomainDev &D = b->doms[d];
     if (!b->active_h.empty() && !b->active_h[d]) continue;
@@ -320,6 +320,7 @@ static MultiTiling multi_tiles(const lbm_batch *b) {
     pery = pery || D.per[1];
     solids = solids || !b->solid[d].empty();
     cells += (long long)D.nx * D.ny;
+    if (D.per[1] && D.ny < 16) low += (long long)D.nx * D.ny;
   }
   if (!cells) return out;
   for (int d = 0; d < b->ndom; ++d) {
@@ -329,14 +330,25 @@ static MultiTiling multi_tiles(const lbm_batch *b) {
   }
   out.plan = multi2d_plan({nx, ny, cells, b->esize, true, pery, solids, FORCE_NONE});
   if (out.plan.steps < 2) return out;
+  const int cap = multi2d_cap(b->esize, true);
+  // the same channels, periodic: 6 steps 37 us, one per launch 32, 3 steps 31
+  if (2 * low > cells) out.plan.steps = std::min(out.plan.steps, 3);
   for (int d = 0; d < b->ndom; ++d) {
     if (!b->active_h.empty() && !b->active_h[d]) continue;
     const DomainDev &D = b->doms[d];
     const std::vector<uint8_t> &cc = b->cclass[d];
-    const int cols = (D.nx + out.plan.tw - 1) / out.plan.tw, rows = (D.ny + out.plan.th - 1) / out.plan.th;
+    // A domain lower than the tile takes wider ones of the same size at most
+    // (300 channels of 500 to 1500 x 4 to 8 cells beside one of 300 x 200, FP32:
+    // 48 us a step with the plan's width, 38 one step per launch, 35 so).
+    int tw = out.plan.tw;
+    while (2 * tw * D.ny <= out.plan.tw * out.plan.th && tw < D.nx &&
+           multi2d_slots(2 * tw, D.ny, out.plan.steps) <= cap &&
+           multi2d_exact(multi2d_slots(2 * tw, D.ny, out.plan.steps), 2 * (tw + out.plan.steps)))
+      tw *= 2;
+    const int cols = (D.nx + tw - 1) / tw, rows = (D.ny + out.plan.th - 1) / out.plan.th;
     // widths in whole groups of 16 cells, so that rows start on the same
     // part of a line
-    const int w = std::min(out.plan.tw, ((D.nx + cols - 1) / cols + 15) / 16 * 16), h = (D.ny + rows - 1) / rows;
+    const int w = std::min(tw, ((D.nx + cols - 1) / cols + 15) / 16 * 16), h = (D.ny + rows - 1) / rows;
     for (int y0 = 0; y0 < D.ny; y0 += h)
       for (int x0 = 0; x0 < D.nx; x0 += w) {
         const MultiTile t{d, x0, y0, std::min(w, D.nx - x0), std::min(h, D.ny - y0)};

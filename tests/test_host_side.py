@@ -227,3 +227,32 @@ since = count()
 lat.step(24)
 assert len(launches("k_step", since)) == 24
 """)
+
+
+@pytest.mark.parametrize("storage,esize", [("f32", 4), ("f64", 8), ("f16", 2)])
+@pytest.mark.parametrize("periodic", [False, True])
+def test_low_domains_in_a_batch(stand_in, storage, esize, periodic):
+    """Domains of few rows beside one of many: their tiles are as large as the
+    others (not as wide), every tile fits the LDS, and all cells are covered."""
+    run(stand_in, TILES + f"""
+class MultiTile(ct.Structure):
+    _fields_ = [(n, ct.c_int) for n in ("d", "x0", "y0", "w", "h")]
+wall = ("wall", None, 1.0)
+faces = {{}} if {periodic} else {{"-x": ("velocity_zh", (0.01, 0.0), 1.0), "+x": ("pressure_abb", None, 1.0), "-y": wall, "+y": wall}}
+rng = np.random.default_rng(0)
+shapes = [(int(rng.integers(500, 1500)), int(rng.integers(3, 9))) for _ in range(200)] + [(300, 200), (3, 3), (40, 500)]
+b = capi.Batch([{{"shape": s, "omega": 1.2, "faces": faces}} for s in shapes], storage="{storage}")
+b.run(50, 0.0, 50)
+a = multi2d()[0]
+cap = (80 * 1024 - 256) // (9 * {esize} + 2) // 16 * 16
+assert a.steps <= 3 or not {periodic}
+tiles = (MultiTile * a.ntiles).from_address(a.tiles)
+seen = [np.zeros(s[::-1], int) for s in shapes]
+for t in tiles:
+    nx, ny = shapes[t.d]
+    seen[t.d][t.y0:t.y0 + t.h, t.x0:t.x0 + t.w] += 1
+    assert slots(t.x0, t.x0 + t.w - 1, t.y0, t.y0 + t.h - 1, nx, ny, a.steps, {periodic}, {periodic}, not {periodic}) <= cap
+    if ny < 9 and nx > 500 and t.x0 + t.w < nx:
+        assert t.w >= 64, (nx, ny, t.w)
+assert all((s == 1).all() for s in seen)
+""")

@@ -57,3 +57,27 @@ def test_low_domains_equal_single_steps(storage, faces):
             out.append(lat.populations())
             lat.close()
         assert np.isfinite(out[0]).all() and np.array_equal(*out), (nx, ny)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage", ["f32", "f64", "f16"])
+@pytest.mark.parametrize("periodic", [False, True])
+def test_batch_of_low_domains_equals_domains_alone(storage, periodic):
+    """Wide tiles in domains of few rows, beside one of many rows."""
+    from lbm_amd import capi
+
+    faces = {} if periodic else {"-x": ("velocity_zh", (0.03, 0.0), 1.0), "+x": ("pressure_abb", None, 1.0), "-y": WALL, "+y": WALL}
+    rng = np.random.default_rng(1)
+    shapes = [(int(rng.integers(500, 1500)), int(rng.integers(3, 9))) for _ in range(30)] + [(300, 200), (3, 3)]
+    fields = [start(s, k) for k, s in enumerate(shapes)]
+    b = capi.Batch([{"shape": s, "omega": 1.1, "faces": faces} for s in shapes], storage=storage)
+    b.init(np.concatenate([f[0] for f in fields]), np.concatenate([f[1] for f in fields]))
+    b.run(20, 0.0, 40)
+    for k in (0, 1, 5, 17, 29, 30, 31):
+        lat = capi.Lattice(shapes[k], storage=storage, omega=1.1, faces=faces)
+        lat.init(*fields[k])
+        for _ in range(40):
+            lat.step(1)
+        assert np.array_equal(b.populations(k), lat.populations()), shapes[k]
+        lat.close()
+    b.close()
