@@ -248,11 +248,12 @@ cap = (80 * 1024 - 256) // (9 * {esize} + 2) // 16 * 16
 assert a.steps <= 3 or not {periodic}
 tiles = (MultiTile * a.ntiles).from_address(a.tiles)
 seen = [np.zeros(s[::-1], int) for s in shapes]
+most = max(t.w * t.h for t in tiles)
 for t in tiles:
     nx, ny = shapes[t.d]
     seen[t.d][t.y0:t.y0 + t.h, t.x0:t.x0 + t.w] += 1
     assert slots(t.x0, t.x0 + t.w - 1, t.y0, t.y0 + t.h - 1, nx, ny, a.steps, {periodic}, {periodic}, not {periodic}) <= cap
-    if ny < 9 and nx > 500 and t.x0 + t.w < nx:
-        assert t.w >= 64, (nx, ny, t.w)
+    if ny < 9 and nx > 500 and t.x0 + t.w < nx:  # twice as wide: larger than the largest, or than the LDS
+        assert 2 * t.w * ny > most or (2 * t.w + 2 * a.steps) * (ny + 2 * a.steps) + 4 * a.steps > cap, (nx, ny, t.w)
 assert all((s == 1).all() for s in seen)
 """)
