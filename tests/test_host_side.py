@@ -253,7 +253,9 @@ for t in tiles:
     nx, ny = shapes[t.d]
     seen[t.d][t.y0:t.y0 + t.h, t.x0:t.x0 + t.w] += 1
     assert slots(t.x0, t.x0 + t.w - 1, t.y0, t.y0 + t.h - 1, nx, ny, a.steps, {periodic}, {periodic}, not {periodic}) <= cap
-    if ny < 9 and nx > 500 and t.x0 + t.w < nx:  # twice as wide: larger than the largest, or than the LDS
-        assert 2 * t.w * ny > most or (2 * t.w + 2 * a.steps) * (ny + 2 * a.steps) + 4 * a.steps > cap, (nx, ny, t.w)
+    if ny < 9 and nx > 500 and t.x0 + t.w < nx:  # twice as wide: larger than the largest, the LDS or the kernel's division allow
+        w = 2 << (t.w - 1).bit_length()  # (the domain is cut evenly into widths of up to a power of two)
+        n = (w + 2 * a.steps) * (ny + 2 * a.steps) + 4 * a.steps
+        assert w * ny > most or n > cap or n * (w + 2 * a.steps) >= 1 << 20, (nx, ny, t.w)
 assert all((s == 1).all() for s in seen)
 """)
