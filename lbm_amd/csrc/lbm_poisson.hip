@@ -513,6 +513,9 @@ static void launch_step(lbm_poisson *h) {
 //   D2Q9 512^2    32 x 16, 4        3.6    16 x 32, 4   3.7      9.9
 //   D2Q9 4096^2   16 x 24, 6        156    32 x 16, 4   176      489
 //   D1Q3 100000   512, 48           0.64   512, 16      0.75     4.7
+// A window lower than the tile takes wider ones of the same size at most, as far
+// as rim holds their lines (its region has the window's rows): 1000000 x 5 D2Q5
+// @P5@.
 static PMulti multi_plan(const lbm_poisson *h) {
   constexpr int NCU = 256;
   const long long cells = (long long)h->nx * h->ny;
@@ -521,18 +524,22 @@ static PMulti multi_plan(const lbm_poisson *h) {
   int lg = 6;
   while (lg < 9 && ((long long)NCU << lg) < cells) ++lg;
   if (h->Q == 3) {
-    m.tw = std::min(1 << lg, h->nx);
+    m.tw = 1 << lg;
     m.th = 1;
     m.steps = 48;
   } else if (cells > 2ll * NCU << 9) {
-    m.tw = std::min(16, h->nx);
-    m.th = std::min(24, h->ny);
+    m.tw = 16;
+    m.th = 24;
     m.steps = 6;
   } else {
-    m.tw = std::min(1 << (lg + 1) / 2, h->nx);
-    m.th = std::min(1 << lg / 2, h->ny);
+    m.tw = 1 << (lg + 1) / 2;
+    m.th = 1 << lg / 2;
     m.steps = lg < 9 ? 8 : 4;
   }
+  const int size = m.tw * m.th;
+  m.th = std::min(m.th, h->ny);
+  while (2 * m.tw * m.th <= size && 2 * (m.tw + m.steps) <= MULTI_RIM && 2 * (m.tw + m.steps) * m.th <= MULTI_CELLS) m.tw *= 2;
+  m.tw = std::min(m.tw, h->nx);
   m.ntx = (h->nx + m.tw - 1) / m.tw;
   m.ntiles = m.ntx * ((h->ny + m.th - 1) / m.th);
   return m;

@@ -17,7 +17,8 @@ int si_capturing = 0;
 #define RECORDS 4096
 int si_launches = 0;
 char si_name[RECORDS][64];
-unsigned char si_args[RECORDS][512]; /* the first argument of a launch */
+unsigned char si_args[RECORDS][512];  /* the first argument of a launch */
+unsigned char si_args2[RECORDS][64]; /* and the second of k_poisson_multi */
 
 static struct { const void *f; char name[64]; } kernels[4096];
 static int nkernels;
@@ -102,6 +103,7 @@ int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t shmem
   if (si_launches < RECORDS) {
     strcpy(si_name[si_launches], name);
     if (strstr(name, "k_multi")) memcpy(si_args[si_launches], args[0], 216);
+    if (strstr(name, "k_poisson_multi")) memcpy(si_args2[si_launches], args[1], 40);
   }
   ++si_launches;
   return 0;

@@ -259,3 +259,40 @@ for t in tiles:
         assert w * ny > most or n > cap or n * (w + 2 * a.steps) >= 1 << 20, (nx, ny, t.w)
 assert all((s == 1).all() for s in seen)
 """)
+
+
+@pytest.mark.parametrize("q", [5, 9])
+def test_low_poisson_windows(stand_in, q):
+    """Windows of few rows: every tile's region fits the LDS and its lines the
+    first-layer arrays, and where there are cells enough a tile holds at least
+    half as many as that of a square window."""
+    run(stand_in, f"""
+class PMulti(ct.Structure):  # lbm_poisson.hip
+    _fields_ = [(n, ct.c_int) for n in ("steps", "tw", "th", "ntx", "ntiles")] + [("phi_prev", ct.c_void_p), ("write_phi", ct.c_int)]
+args = (ct.c_ubyte * 64 * 4096).in_dll(si, "si_args2")
+def extent(b, e, back, n):
+    return max(min(b, n - 3) - back, 0), min(max(e, 2) + back, n - 1)
+def plan(nx, ny):
+    p = poisson.Poisson({q}, nx, ny, 1.0, 0.0)
+    p.set_faces({{f: ("neumann", None, k) for k, f in enumerate(("-x", "+x", "-y", "+y"))}})
+    p.init(np.zeros(nx * ny))
+    since = count()
+    p.step(48)
+    p.close()
+    return PMulti.from_buffer_copy(bytes(args[since])[:40])
+for cells in (400, 20000, 100000, 400000, 2000000):
+    side = int(cells ** 0.5)
+    square = plan(side, side)
+    for ny in list(range(5, 27)) + [40]:
+        nx = max(5, cells // ny)
+        m = plan(nx, ny)
+        assert m.ntx == -(-nx // m.tw) and m.ntiles == m.ntx * -(-ny // m.th)
+        for x0 in {{0, m.tw if m.tw < nx else 0, (nx - 1) // m.tw * m.tw}}:
+            for y0 in range(0, ny, m.th):
+                x = extent(x0, min(x0 + m.tw, nx) - 1, m.steps, nx)
+                y = extent(y0, min(y0 + m.th, ny) - 1, m.steps, ny)
+                pitch, rows = x[1] - x[0] + 1, y[1] - y[0] + 1
+                assert pitch * rows <= 1024 and pitch <= 128 and rows <= 128, (nx, ny, m.tw, m.th, m.steps)
+        if cells >= 100000:
+            assert 2 * m.tw * m.th > square.tw * square.th or m.th < ny or 2 * (m.tw + m.steps) > 128, (nx, ny, m.tw, m.th)
+""")

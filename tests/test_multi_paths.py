@@ -81,3 +81,24 @@ def test_batch_of_low_domains_equals_domains_alone(storage, periodic):
         assert np.array_equal(b.populations(k), lat.populations()), shapes[k]
         lat.close()
     b.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["dirichlet", "neumann"])
+@pytest.mark.parametrize("Q,nx,ny", [(5, 100003, 5), (9, 66661, 6), (5, 60011, 8), (9, 50001, 13), (5, 900001, 5), (9, 31, 5)])
+def test_low_poisson_windows_equal_single_steps(Q, nx, ny, kind):
+    from lbm_amd import poisson
+
+    rng = np.random.default_rng(ny)
+    faces = {f: (kind if f[1] == "y" else "dirichlet", rng.random(ny if f[1] == "x" else nx), k)
+             for k, f in enumerate(("-x", "+x", "-y", "+y"))}
+    phi0, out = rng.random(nx * ny), []
+    for calls in ((13, 2, 9), (1,) * 24):
+        p = poisson.Poisson(Q, nx, ny, 1.3, -0.003)
+        p.set_faces(faces)
+        p.init(phi0)
+        for n in calls:
+            p.step(n)
+        out.append((p.phi(), p.step_check()[0]))
+        p.close()
+    assert np.isfinite(out[0][0]).all() and np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
