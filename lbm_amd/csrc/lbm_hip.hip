@@ -577,13 +577,18 @@ static int multi3d_fit(const lbm_handle *h) {
 
 // The two-step kernel's tiles, and its blocks that meet a solid.  Their number
 // depends on the storage form (the tile does), so the array holds the most of
-// any.  The handle takes the plan last: without room for the array, or where
-// the launch that fills it fails, it has none and the steps run one per launch.
+// any.  The handle takes the plan last: where single steps are faster, without
+// room for the array, or where the launch that fills it fails, it has none and
+// the steps run one per launch.
 static void build_solid3(lbm_handle *h) {
   const int cls = multi3d_fit(h);
   h->plan3 = Multi3dPlan{};
   if (cls == MULTI3D_NONE) return;
   const Multi3dPlan plan = multi3d_plan(h->nx, h->ny, h->nz, h->esize, cls);
+  dim3 g, b;
+  launch_dims(h, g, b);
+  const double lanes = (double)g.x * b.x * ((double)g.y * b.y) * g.z;
+  if (multi3d_ratio(plan, h->nx, h->ny, h->nz, h->esize, cls, h->face, h->has_flags, force_kind(h->F), lanes) > 0.99) return;
   if (h->has_flags) {
     if (!h->solid3) {
       long long n = 0;

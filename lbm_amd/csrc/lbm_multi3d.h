@@ -20,17 +20,15 @@ enum : int {
 // 128 cavity FP32 126 against 136 us a step).
 constexpr int multi3d_threads(int esize, int cls) { return cls == MULTI3D_WALLS && esize != 8 ? 256 : 512; }
 
-// Two steps in one pass take longer than two launches (microseconds per step,
-// this kernel against single steps)
-//  - with too few columns to fill the chip: FP32 box of 64^3 9.9 against 8.6,
-//    of 128^3 49 against 59; FP32 cavity of 128 x 64 x 64 20.5 against 19.6,
-//    of 160 x 96 x 96 54 against 71; FP64 box of 40^3 6.6 against 6.7, of 52^3
-//    8.1 against 11; FP64 cavity of 50^3 15.4 against 12.2, of 97 x 61 x 45
-//    20.4 against 21.4; FP16 box of 128^3 37 against 33, of 150^3 63 against 86;
-//  - in 16-bit storage with walls, where the masks cost more than the halved
-//    traffic (512 x 128 x 128 sphere channel 187 against 181);
-//  - in FP32 with NEEM faces, whose FP64 arithmetic is done for the halo too
-//    (the same channel 289 against 249; FP64 of 300 x 200 x 101 258 against 437).
+// Two steps in one pass take longer than two launches with too few columns to
+// fill the chip (microseconds per step, this kernel against single steps: FP32
+// box of 64^3 9.9 against 8.6; FP32 cavity of 128 x 64 x 64 20.5 against 19.6;
+// FP16 box of 128^3 37 against 33; FP64 box of 40^3 6.6 against 6.7; FP64 cavity of
+// 50^3 15.4 against 12.2), in 16-bit storage with walls, where the masks cost
+// more than the halved traffic (512 x 128 x 128 sphere channel 187 against 181),
+// and in FP32 with NEEM faces, whose FP64 arithmetic is done for the halo too
+// (the same channel 289 against 249; FP64 of 300 x 200 x 101 258 against 437).
+// Beyond these bounds multi3d_ratio decides.
 inline int multi3d_class(const FaceDev *face, bool solids, long long cells, int esize) {
   int c = solids ? MULTI3D_WALLS : MULTI3D_BOX;
   for (int f = 0; f < 6; ++f) {
@@ -62,8 +60,14 @@ struct Multi3dArgs {
 
 struct Multi3dPlan {
   int tw, ntx, nty, slabs;
+  double cost;  // planes that the busiest CU works through
 };
 Multi3dPlan multi3d_plan(int nx, int ny, int nz, int esize, int cls);
+
+// Time of the two-step kernel over that of single steps.  lanes: threads of a
+// single-step launch, force: a force_kind.
+double multi3d_ratio(const Multi3dPlan &p, int nx, int ny, int nz, int esize, int cls, const FaceDev *face, bool solids,
+                     int force, double lanes);
 
 // solid[0 .. ntx * nty * slabs) of the plan in a, from a.links
 void multi3d_solid(const Multi3dArgs &a, unsigned char *solid, hipStream_t s);

@@ -20,6 +20,7 @@
 #include "lbm_multi3d.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace lbm {
 
@@ -397,6 +398,7 @@ Multi3dPlan multi3d_plan(int nx, int ny, int nz, int esize, int cls) {
       if (least == 0.0 || cost < (p.tw == best.tw ? 1.0 : 0.8) * least) {
         least = cost;
         best = p;
+        best.cost = cost;
       }
     }
   };
@@ -404,6 +406,52 @@ Multi3dPlan multi3d_plan(int nx, int ny, int nz, int esize, int cls) {
   if (esize == 8 && 2ll * 19 * esize * nx * ny * nz <= CACHE)
     for (int n = (nx + 63) / 64; n <= (nx + 15) / 16; ++n) width((nx + n - 1) / n);
   return best;
+}
+
+// FP64 storage halves its traffic and hardly adds to its arithmetic: two steps
+// win on every domain above multi3d_class's bounds but those with walls, beyond
+// the cache and a few rows high (1024 x 4 x 1024 1.17 times as long, 512 x 5 x 400
+// with NEEM faces 1.08).  In FP32 and 16-bit storage the second step's arithmetic,
+// for the halo too, takes up much of what the traffic gives.  The logarithm of
+// the ratio is fitted, closely where it is near zero, to 950 pairs of timings:
+// idle lanes of the single step (its rows are rounded up to its blocks), the
+// planes a CU works through here per cell, the body force (a general one costs
+// a quarter: FP16 box of 256^3 232 us a step single; two steps 200, with a force
+// along x 219, along y 278), solids and walls across x (single steps slow down
+// more), moving walls (256 x 128 x 128 with three of them 135 single, 170; with
+// none 121 single, 114).  Of the 700 pairs of at least 20 cells each way 6 are
+// more than 3 % slower than single steps, the worst 9 %.  In three or four rows
+// most of a block's threads idle (1024 x 3 x 1024 FP32 box 85 single, 114).
+double multi3d_ratio(const Multi3dPlan &p, int nx, int ny, int nz, int esize, int cls, const FaceDev *face, bool solids,
+                     int force, double lanes) {
+  const double cells = (double)nx * ny * nz, idle = std::log(cells / lanes);
+  if (esize == 8)
+    return cls == MULTI3D_WALLS && !solids && ny < 6 && idle > -0.4 && 2 * 19 * 8 * cells > (double)(256 << 20) ? 1.1 : 0.9;
+  if (ny < (solids ? 4 : 5)) return 1.1;
+  // (beyond a wall there is no plane to take the first step of)
+  const double beyond = p.slabs == 1 && face[4].kind != LBM_FACE_PERIODIC ? (double)nz / (nz + 1) : 1.0;
+  const double planes = std::log(p.cost * beyond * 131072.0 / cells),
+               mb = std::log(cells * esize * 38 / (1 << 20));
+  if (esize == 2) {
+    const double f[3] = {0.0, 0.104, 0.243};
+    return std::exp(0.055 + 0.576 * idle + 0.27 * planes - 0.048 * mb + f[force]);
+  }
+  if (cls == MULTI3D_BOX) {
+    const double f[3] = {0.0, 0.022, 0.083};
+    return std::exp(-0.526 + 0.449 * idle + 0.148 * planes + 0.041 * mb + 0.184e6 / cells + f[force]);
+  }
+  int moving = 0;
+  bool movx = false, movy = false;
+  for (int i = 0; i < 6; ++i) {
+    if (face[i].kind != LBM_FACE_WALL || (face[i].u[0] == 0.0 && face[i].u[1] == 0.0 && face[i].u[2] == 0.0)) continue;
+    ++moving;
+    movx = movx || i < 2;
+    movy = movy || i == 2 || i == 3;
+  }
+  const double f[3] = {0.0, 0.051, 0.122};
+  return std::exp(-0.507 + 0.476 * idle + 0.504 * planes - 0.033 * mb + f[force] - (solids ? 0.219 : 0.0) -
+                  (face[0].kind != LBM_FACE_PERIODIC ? 0.346 / ((nx + 63) / 64) : 0.0) +
+                  (movx ? 0.208 : movy ? 0.08 : 0.0) + 0.056 * std::max(0, moving - 1));
 }
 
 void multi3d_solid(const Multi3dArgs &a, unsigned char *solid, hipStream_t s) {

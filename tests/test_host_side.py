@@ -296,3 +296,39 @@ for cells in (400, 20000, 100000, 400000, 2000000):
         if cells >= 100000:
             assert 2 * m.tw * m.th > square.tw * square.th or m.th < ny or 2 * (m.tw + m.steps) > 128, (nx, ny, m.tw, m.th)
 """)
+
+
+# domains whose two steps in one pass were timed above or below two launches
+TWO_STEP_ROUTES = """
+wall = ("wall", None, 1.0)
+moving = ("wall", (0.01, 0.02, 0.01), 1.0)
+channel = {"-y": wall, "+y": wall, "-z": wall, "+z": wall}
+box = dict(channel, **{"-x": wall, "+x": wall})
+def two_steps(shape, storage, faces, force=(0.0, 0.0, 0.0), solids=0.0):
+    solid = (np.random.default_rng(0).random(np.prod(shape)) < solids).astype(np.uint8) if solids else None
+    lat = capi.Lattice(shape, storage=storage, omega=1.2, faces=faces, force=force, solid=solid)
+    since = count()
+    lat.step(2)
+    lat.close()
+    names = [n for n, _ in launches("", since)]
+    assert len(names) in (1, 2) and ("k_multi3d" in names[0]) == (len(names) == 1), names
+    return len(names) == 1
+x, xy = (1e-6, 0.0, 0.0), (1e-6, 1e-6, 0.0)
+"""
+
+
+def test_two_steps_only_where_they_are_faster(stand_in):
+    run(stand_in, TWO_STEP_ROUTES + """
+for shape, storage, faces, force, solids, two in (
+        ((160, 96, 96), "f32", channel, x, 0.0, True), ((100, 100, 100), "f32", channel, x, 0.0, False),
+        ((130, 101, 99), "f32", box, xy, 0.0, True), ((128, 96, 96), "f32", channel, xy, 0.0, False),
+        ((128, 96, 96), "f32", dict(box, **{"+y": moving}), (0.0,) * 3, 0.0, True),
+        ((128, 96, 96), "f32", dict(box, **{"+x": moving, "+y": moving, "+z": moving}), (0.0,) * 3, 0.0, False),
+        ((100, 100, 100), "f32", channel, x, 0.2, True),
+        ((128, 128, 128), "f32", {}, xy, 0.0, True), ((128, 64, 66), "f32", {}, (0.0,) * 3, 0.0, False),
+        ((512, 3, 400), "f32", {}, (0.0,) * 3, 0.0, False), ((512, 3, 400), "f64", {}, (0.0,) * 3, 0.0, True),
+        ((256, 128, 100), "f16", {}, (0.0,) * 3, 0.0, True), ((256, 128, 100), "f16", {}, xy, 0.0, False),
+        ((512, 6, 1100), "f16", {}, (0.0,) * 3, 0.0, False), ((512, 5, 400), "f64", channel, (0.0,) * 3, 0.0, False),
+        ((97, 61, 45), "f64", box, (0.0,) * 3, 0.0, True)):
+    assert two_steps(shape, storage, faces, force, solids) == two, (shape, storage, faces, force, solids)
+""")
