@@ -23,11 +23,13 @@ constexpr int multi3d_threads(int esize, int cls) { return cls == MULTI3D_WALLS 
 // Two steps in one pass take longer than two launches with too few columns to
 // fill the chip (microseconds per step, this kernel against single steps: FP32
 // box of 64^3 9.9 against 8.6; FP32 cavity of 128 x 64 x 64 20.5 against 19.6;
-// FP16 box of 128^3 37 against 33; FP64 box of 40^3 6.6 against 6.7; FP64 cavity of
-// 50^3 15.4 against 12.2), in 16-bit storage with walls, where the masks cost
-// more than the halved traffic (512 x 128 x 128 sphere channel 187 against 181),
-// and in FP32 with NEEM faces, whose FP64 arithmetic is done for the halo too
-// (the same channel 289 against 249; FP64 of 300 x 200 x 101 258 against 437).
+// FP16 box of 128^3 37 against 33; FP64 box of 40^3 6.6 against 6.7; FP64 walls of
+// 128 x 32 x 32 9.7 against 8.3, of 256 x 24 x 25 with NEEM faces 1.2 times as
+// long, of 128 x 38 x 36 the same; of 24 domains from 131072 to 262144 cells those
+// above 196608 all gain, 1 to 37 %), in 16-bit storage with walls, where the masks
+// cost more than the halved traffic (512 x 128 x 128 sphere channel 187 against
+// 181), and in FP32 with NEEM faces, whose FP64 arithmetic is done for the halo
+// too (the same channel 289 against 249; FP64 of 300 x 200 x 101 258 against 437).
 // Beyond these bounds multi3d_ratio decides.
 inline int multi3d_class(const FaceDev *face, bool solids, long long cells, int esize) {
   int c = solids ? MULTI3D_WALLS : MULTI3D_BOX;
@@ -38,7 +40,7 @@ inline int multi3d_class(const FaceDev *face, bool solids, long long cells, int 
       return MULTI3D_NONE;
     c = MULTI3D_WALLS;
   }
-  const long long least = esize == 8 ? (c == MULTI3D_WALLS ? 1ll << 18 : 1ll << 17)
+  const long long least = esize == 8 ? (c == MULTI3D_WALLS ? 3ll << 16 : 1ll << 17)
                           : esize == 4 ? (c == MULTI3D_WALLS ? 3ll << 18 : 1ll << 19)
                                        : (c == MULTI3D_WALLS ? 1ll << 62 : 3ll << 20);
   return cells > least ? c : MULTI3D_NONE;

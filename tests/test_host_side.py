@@ -332,3 +332,11 @@ for shape, storage, faces, force, solids, two in (
         ((97, 61, 45), "f64", box, (0.0,) * 3, 0.0, True)):
     assert two_steps(shape, storage, faces, force, solids) == two, (shape, storage, faces, force, solids)
 """)
+
+
+def test_least_cells_of_two_steps_in_fp64(stand_in):
+    run(stand_in, TWO_STEP_ROUTES + """
+for shape, two in (((64, 64, 48), False), ((64, 64, 49), True), ((700, 20, 18), True), ((128, 38, 36), False)):
+    for faces in (channel, box):
+        assert two_steps(shape, "f64", faces) == two, shape
+""")
