@@ -2,16 +2,17 @@
 
 Workload (N=1): 256^3 periodic box, D3Q19 BGK, tau = 0.6, FP32 populations
 (stored shifted, f - w), Taylor-Green vortex u0 = 0.05 plus seeded Gaussian
-noise sigma = 1e-3, rho = 1.  A step is one fused collide+stream launch over
-all 16.8M cells.  W warm-up steps, untimed settling groups until the step
+noise sigma = 1e-3, rho = 1.  A step updates all 16.8M cells (fused collide
+and stream).  W warm-up steps, untimed settling groups until the step
 time is stable (reported in "settle"), then K timed steps bracketed by
 synchronisation, run without a break as five repetitions with HIP events
 recorded between them on the stream the kernel is launched on; the reported
 time per step is the median over the repetitions (min, max and the mean
 over all K steps beside it).
 
-Algorithmic bytes per lattice update: 2 * 19 * 4 = 152 B (one read and one
-write of every population); achieved = 152 B * cells / launch time.
+Algorithmic bytes per launch: 2 * 19 * 4 = 152 B per cell (one read and one
+write of every population), whatever steps the launch takes (two, here);
+achieved = 152 B * cells / launch time, and beside it the same per update.
 The CPU baseline is the project's FP64 oracle (OpenMP) on a bounded sample
 of the same workload (64^3 cells, a few steps), run on this host.
 
@@ -145,8 +146,9 @@ def run_batch(args):
             "steps_min": int(steps[steps > 0].min()) if (steps > 0).any() else None,
             "steps_max": int(steps.max()), "updates": updates, "GLUPS_effective": round(glups, 2),
             "GLUPS_all_cells": round(glups_all, 2),
-            "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                         "frac": round(achieved / PEAK_HBM_GBS, 4)},
+            # the bytes of every update over the time: launches take several
+            # steps, so memory moves fewer
+            "per_update": {"bytes": 2 * 9 * bpp + 1, "achieved": round(achieved, 1), "unit": "GB/s"},
             "tiling": {"tile_x": tx, "blocks": blocks, "one_launch": one, "tuning_s": round(tune_s, 2),
                        "ms_per_step_full": tms},
             "tiles": info["tiles"]}
@@ -372,9 +374,10 @@ def run_poisson(args):
                       "ms_per_step": round(ms, 5), "steps": args.steps, "warmup": args.warmup,
                       "higher_is_better": True, "dtype": "f64", "data": "synthetic (Dirichlet box, phi = 1 on the faces)",
                       "config": {"workload": f"D2Q9 Poisson {n}x{n}, tau 1, Debye-Hueckel kappa 27.79"},
-                      "roofline": {"bound": "hbm", "achieved": round(alg / (ms * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBS,
-                                   "unit": "GB/s", "frac": round(alg / (ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
-                                   "alg_bytes_per_launch": alg},
+                      # the bytes of every update over the time: launches take
+                      # several steps, so memory moves fewer
+                      "per_update": {"bytes": 2 * 9 * 8 + 8, "achieved": round(alg / (ms * 1e-3) / 1e9, 1),
+                                     "unit": "GB/s"},
                       "residual_last": res}), flush=True)
 
 
@@ -494,13 +497,14 @@ def main():
     mlups = cells / (ms_per_step * 1e-3) / 1e6
     bpp = capi.BYTES[args.storage]
     alg_bytes = 2 * 19 * bpp * cells
-    achieved = alg_bytes / (ms_per_step * 1e-3) / 1e9
+    # a launch reads and writes every population once, whatever steps it takes:
+    # `achieved` is the rate at which memory has to move these bytes, and
+    # "per_update" the bytes of every update over the time, the rate that one
+    # step per launch would need
+    per_launch = lat.steps_per_launch(max(groups))
+    achieved = alg_bytes / (ms_per_step * per_launch * 1e-3) / 1e9
     s = lat.reduce()
     lat.close()
-    # plain steps of a box this large run two per launch (multi3d_class in
-    # lbm_multi3d.h): a launch needs alg_bytes once, so `frac`, the bytes of
-    # every update over the time, is of the rate one step per launch could reach
-    two = args.halo == "l2" and cells > {8: 1 << 17, 4: 1 << 19, 2: 3 << 20}[bpp]
     # the committed counter run covers the default (L2 gather) kernel only
     traffic = load_traffic(f"traffic_d3q19_{args.storage}_{n}.json") if args.halo == "l2" else None
     line = {
@@ -522,7 +526,9 @@ def main():
                    "gather": args.halo},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(achieved / PEAK_HBM_GBS, 4), "traffic": traffic,
-                     "alg_bytes_per_launch": alg_bytes, "steps_per_launch": 2 if two else 1},
+                     "alg_bytes_per_launch": alg_bytes, "steps_per_launch": per_launch,
+                     "per_update": {"bytes": 2 * 19 * bpp, "achieved": round(achieved * per_launch, 1),
+                                    "frac": round(achieved * per_launch / PEAK_HBM_GBS, 4)}},
         "timing": {"repetitions": len(groups), "steps_per_repetition": groups,
                    "ms_per_step_median": round(ms_per_step, 5), "ms_per_step_min": round(float(per_step.min()), 5),
                    "ms_per_step_max": round(float(per_step.max()), 5),

@@ -149,6 +149,11 @@ int lbm_init_fields(lbm_handle *h, const double *rho, const double *u);
 /* Advance nsteps time steps (LBMSolver::timeStep, src/lbm/solver.cpp:307-320). */
 int lbm_step(lbm_handle *h, int32_t nsteps);
 
+/* The most steps a launch of lbm_step(h, nsteps) takes: more than one where
+ * the lattice's faces, size and storage let several go in one pass over
+ * memory and that is faster.  The results do not depend on it. */
+int lbm_steps_per_launch(const lbm_handle *h, int32_t nsteps, int32_t *steps);
+
 /* Advance two steps; the second reports the one-step change of the
  * macroscopic fields plus mass and momentum (convergenceCondition,
  * src/lbm/solver.cpp:233-263).  Returns LBM_DIVERGED if NaN/Inf appear. */

@@ -48,7 +48,7 @@ class Sums(ct.Structure):
 
 
 # every symbol declared in include/lbm_hip.h
-EXPORTS = ["lbm_create", "lbm_set_bc", "lbm_init_fields", "lbm_step", "lbm_step_check", "lbm_step_ex", "lbm_step_ex_noalloc",
+EXPORTS = ["lbm_create", "lbm_set_bc", "lbm_init_fields", "lbm_step", "lbm_steps_per_launch", "lbm_step_check", "lbm_step_ex", "lbm_step_ex_noalloc",
            "lbm_get_macros",
            "lbm_reduce", "lbm_get_populations", "lbm_set_populations", "lbm_time_steps", "lbm_time_step_groups", "lbm_set_launch",
            "lbm_set_halo", "lbm_set_pressure_forcing", "lbm_set_index_width", "lbm_set_storage", "lbm_info", "lbm_synchronize", "lbm_destroy", "lbm_last_error", "lbm_copy_bench"]
@@ -70,6 +70,7 @@ def load():
     lib.lbm_set_bc.argtypes = [P, ct.POINTER(BcDesc), ct.c_int32]
     lib.lbm_init_fields.argtypes = [P, dp, dp]
     lib.lbm_step.argtypes = [P, ct.c_int32]
+    lib.lbm_steps_per_launch.argtypes = [P, ct.c_int32, ct.POINTER(ct.c_int32)]
     lib.lbm_step_check.argtypes = [P, ct.POINTER(Sums)]
     lib.lbm_step_ex.argtypes = [P, ct.c_int32, ct.POINTER(Sums)]
     lib.lbm_step_ex_noalloc.argtypes = [P, ct.c_int32, ct.POINTER(Sums)]
@@ -168,6 +169,12 @@ class Lattice:
 
     def step(self, n=1):
         self._check(self.lib.lbm_step(self.h, int(n)))
+
+    def steps_per_launch(self, n):
+        """The most steps a launch of step(n) takes."""
+        k = ct.c_int32()
+        self._check(self.lib.lbm_steps_per_launch(self.h, int(n), ct.byref(k)))
+        return k.value
 
     def step_check(self):
         s = Sums()

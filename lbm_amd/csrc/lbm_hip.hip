@@ -953,14 +953,34 @@ static int multi3d_cls(const lbm_handle *h) {
   return multi3d_fit(h);
 }
 
+static int launches_of(int32_t nsteps, int most) { return nsteps / most + (nsteps % most != 0); }
+
+// The multi-step plan of a call of nsteps plain D2Q9 steps; steps 1: one step
+// per launch.
+static Multi2dPlan plan2d(const lbm_handle *h, int32_t nsteps, int &cls) {
+  cls = nsteps > 1 ? multi2d_cls(h) : MULTI2D_NONE;
+  if (cls == MULTI2D_NONE) return Multi2dPlan{1, 0, 0, false};
+  return multi2d_plan({h->nx, h->ny, h->ncell, h->esize, cls != MULTI2D_BOX, h->per[1] != 0, h->has_flags, force_kind(h->F)});
+}
+
+int lbm_steps_per_launch(const lbm_handle *h, int32_t nsteps, int32_t *steps) {
+  if (!h || nsteps < 1 || !steps) return fail(nullptr, LBM_EINVAL, "lbm_steps_per_launch: bad argument");
+  int cls = 0;
+  const Multi2dPlan p = plan2d(h, nsteps, cls);
+  *steps = nsteps > 1 && multi3d_cls(h) != MULTI3D_NONE ? 2 : 1;
+  if (p.steps > 1) {
+    const int n = launches_of(nsteps, p.steps);
+    *steps = nsteps / n + (nsteps % n != 0);
+  }
+  return LBM_OK;
+}
+
 int lbm_step(lbm_handle *h, int32_t nsteps) {
   if (!h || nsteps < 0) return fail(h, LBM_EINVAL, "lbm_step: bad argument");
-  const int cls = nsteps > 1 ? multi2d_cls(h) : MULTI2D_NONE;
-  Multi2dPlan p{1, 0, 0, false};
-  if (cls != MULTI2D_NONE)
-    p = multi2d_plan({h->nx, h->ny, h->ncell, h->esize, cls != MULTI2D_BOX, h->per[1] != 0, h->has_flags, force_kind(h->F)});
+  int cls = 0;
+  const Multi2dPlan p = plan2d(h, nsteps, cls);
   if (p.steps > 1) {
-    const int n = nsteps / p.steps + (nsteps % p.steps != 0);
+    const int n = launches_of(nsteps, p.steps);
     for (int i = 0; i < n; ++i) {  // as even as possible
       const int rc = launch_multi2d(h, p, cls, nsteps / n + (i < nsteps % n ? 1 : 0));
       if (rc) return rc;

@@ -340,3 +340,21 @@ for shape, two in (((64, 64, 48), False), ((64, 64, 49), True), ((700, 20, 18), 
     for faces in (channel, box):
         assert two_steps(shape, "f64", faces) == two, shape
 """)
+
+
+def test_steps_per_launch(stand_in):
+    """lbm_steps_per_launch against the launches that lbm_step makes."""
+    run(stand_in, """
+wall = ("wall", None, 1.0)
+for shape, storage, faces in (((64, 32), "f64", {}), ((333333, 3), "f16", {}), ((400, 300), "f32", {"-y": wall, "+y": wall}),
+                              ((64, 32), "f32", {"-y": ("wall_eq", None, 1.0), "+y": ("wall_eq", None, 1.0)}),
+                              ((128, 128, 64), "f32", {}), ((40, 40, 40), "f32", {})):
+    lat = capi.Lattice(shape, storage=storage, omega=1.2, faces=faces)
+    for n in (1, 2, 3, 9, 24, 25):
+        since = count()
+        lat.step(n)
+        multi = multi2d(since)
+        most = max(a.steps for a in multi) if multi else 2 if launches("k_multi3d", since) else 1
+        assert lat.steps_per_launch(n) == most, (shape, storage, n, most)
+    lat.close()
+""")
