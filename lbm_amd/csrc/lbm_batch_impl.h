@@ -866,7 +866,7 @@ int lbm_batch_get_macros(lbm_batch *b, int32_t dom, double *rho, double *u) {
   // Small domains of a large batch: the kernel writes pinned memory itself.
   // Otherwise through device staging, kept (allocating it for every domain
   // took half of a read-back).  512 domains of 256 x 128: 35 -> 26 ms.
-  void *pinned = bytes <= Readback::CHUNK && b->ndom >= 8 ? b->out.pinned() : nullptr;
+  void *pinned = bytes <= Readback::CHUNK && b->ndom >= 8 ? b->out.pinned(b->stream) : nullptr;
   if (!pinned && bytes > b->io_cap) {
     if (b->io) BHIPCHK(b, hipFree(b->io));
     b->io = nullptr;

@@ -39,15 +39,20 @@ class Readback {
     return e != hipSuccess ? e : copy(dst2, src2, bytes2, s);
   }
 
-  // CHUNK bytes of pinned memory that a kernel may write and the host reads
-  // once the stream is synchronised; null where there are none
-  void *pinned() { return reserve(1) ? chunk_[0] : nullptr; }
+  // CHUNK bytes of pinned memory that a kernel of stream s may write and the
+  // host reads once the stream is synchronised; null where there are none
+  void *pinned(hipStream_t s) {
+    const OnDevice of(s);
+    return of.ok && reserve(1) ? chunk_[0] : nullptr;
+  }
 
   // bytes from src on the device to dst, after what is queued on the stream;
   // done on return
   hipError_t copy(void *dst, const void *src, size_t bytes, hipStream_t s) {
+    if (bytes < LEAST) return plain(dst, src, bytes, s);
+    const OnDevice of(s);
     const size_t n = (bytes + CHUNK - 1) / CHUNK;
-    if (bytes < LEAST || !reserve(CHUNKS)) return plain(dst, src, bytes, s);
+    if (!of.ok || !reserve(CHUNKS)) return plain(dst, src, bytes, s);
     char *to = static_cast<char *>(dst);
     const char *from = static_cast<const char *>(src);
     std::mutex mu;
@@ -55,9 +60,8 @@ class Readback {
     size_t issued = 0;        // chunks whose transfer is queued
     std::vector<char> empty;  // by chunk: emptied
     hipError_t error = hipSuccess;
-    int device = 0;
     auto work = [&](size_t first, size_t step) {
-      (void)hipSetDevice(device);
+      (void)hipSetDevice(of.device);
       for (size_t k = first; k < n; k += step) {
         {
           std::unique_lock<std::mutex> lock(mu);
@@ -80,7 +84,6 @@ class Readback {
     try {
       empty.assign(n, 0);
       threads.reserve(THREADS);
-      if (hipGetDevice(&device) != hipSuccess) return plain(dst, src, bytes, s);
       for (size_t t = 0; t < std::min<size_t>(THREADS, n); ++t) threads.emplace_back(work, t, std::min<size_t>(THREADS, n));
     } catch (...) {  // no memory or no threads: let those that started go
       {
@@ -124,6 +127,18 @@ class Readback {
   ~Readback() { release(); }
 
  private:
+  // The stream's device is current for the scope's length: events belong to
+  // the device they are made on, and the caller may have another one current.
+  struct OnDevice {
+    int device = 0, before = 0;
+    bool ok;
+    explicit OnDevice(hipStream_t s)
+        : ok(hipStreamGetDevice(s, &device) == hipSuccess && hipGetDevice(&before) == hipSuccess &&
+             (device == before || hipSetDevice(device) == hipSuccess)) {}
+    ~OnDevice() {
+      if (ok && device != before) (void)hipSetDevice(before);
+    }
+  };
   static constexpr size_t LEAST = 16u << 20;  // below, the runtime's copy is as fast
 
   static hipError_t plain(void *dst, const void *src, size_t bytes, hipStream_t s) {

@@ -42,10 +42,14 @@ int hipMemset(void *p, int v, size_t n) { memset(p, v, n); return 0; }
 int hipMemsetAsync(void *p, int v, size_t n, void *st) { (void)st; return hipMemset(p, v, n); }
 int hipGetLastError(void) { int e = last_error; last_error = 0; return e; }
 const char *hipGetErrorString(int e) { return e ? "made to fail" : "no error"; }
-int hipGetDevice(int *d) { *d = 0; return 0; }
-int hipSetDevice(int d) { (void)d; return 0; }
+static __thread int device;
+int hipGetDevice(int *d) { *d = device; return 0; }
+int hipSetDevice(int d) { device = d; return 0; }
 int hipGetSymbolAddress(void **p, const void *s) { (void)s; *p = calloc(1, 256); return 0; }
-int hipStreamCreateWithFlags(void **s, unsigned f) { (void)f; *s = malloc(1); return 0; }
+/* streams and events hold their device */
+static int *on_device(void) { int *p = malloc(sizeof(int)); *p = device; return p; }
+int hipStreamCreateWithFlags(void **s, unsigned f) { (void)f; *s = on_device(); return 0; }
+int hipStreamGetDevice(void *s, int *d) { *d = *(int *)s; return 0; }
 int hipStreamDestroy(void *s) { free(s); return 0; }
 int hipStreamSynchronize(void *s) { (void)s; return 0; }
 int hipStreamBeginCapture(void *s, int m) { (void)s; (void)m; si_capturing = 1; return 0; }
@@ -60,10 +64,10 @@ int hipGraphLaunch(void *e, void *s) {
     if (active[d]) { active[d] = 0; --si_retire; }
   return 0;
 }
-int hipEventCreate(void **e) { *e = malloc(1); return 0; }
+int hipEventCreate(void **e) { *e = on_device(); return 0; }
 int hipEventCreateWithFlags(void **e, unsigned f) { (void)f; return hipEventCreate(e); }
 int hipEventDestroy(void *e) { free(e); return 0; }
-int hipEventRecord(void *e, void *s) { (void)e; (void)s; return 0; }
+int hipEventRecord(void *e, void *s) { return *(int *)e == *(int *)s ? 0 : (last_error = 400); }
 int hipEventSynchronize(void *e) { (void)e; return 0; }
 int hipEventElapsedTime(float *t, void *a, void *b) { (void)a; (void)b; *t = 1.0f; return 0; }
 

@@ -358,3 +358,24 @@ for shape, storage, faces in (((64, 32), "f64", {}), ((333333, 3), "f16", {}), (
         assert lat.steps_per_launch(n) == most, (shape, storage, n, most)
     lat.close()
 """)
+
+
+def test_large_readback_with_another_device_current(stand_in):
+    """A handle's read-backs go on its own device, whichever the caller has
+    current (a read-back of 18 MB goes through events)."""
+    run(stand_in, """
+si.hipSetDevice(1)
+lat = capi.Lattice((1000, 750), storage="f64", omega=1.2)
+b = capi.Batch([{"shape": (1000, 750), "omega": 1.2}], storage="f64")
+p = poisson.Poisson(5, 1600, 1400, 1.0, 0.0)
+p.set_faces({f: ("neumann", None, k) for k, f in enumerate(("-x", "+x", "-y", "+y"))})
+p.init(np.zeros(1600 * 1400))
+si.hipSetDevice(0)
+lat.macros()
+lat.populations()
+b.macros(0)
+p.phi()
+current = ct.c_int()
+si.hipGetDevice(ct.byref(current))
+assert current.value == 0
+""")
