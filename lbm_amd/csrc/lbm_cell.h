@@ -132,17 +132,14 @@ __host__ __device__ constexpr bool leads(int j) {
 }
 
 // 1 / x in FP64: the hardware's estimate, Newton steps and the fix-up of
-// zeros and infinities.  With three steps the same instructions on the same
-// values as the compiler's quotient, without its scaling (which a density
-// never needs); two leave it within an ulp.
-template <int STEPS>
+// zeros and infinities; the same instructions on the same values as the
+// compiler's quotient, without its scaling (which a density never needs).
 __device__ __forceinline__ double reciprocal(double x) {
   double r = __builtin_amdgcn_rcp(x);
 #pragma unroll
-  for (int i = 0; i < STEPS; ++i) r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+  for (int i = 0; i < 3; ++i) r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
   return __builtin_amdgcn_div_fixup(r, x, 1.0);
 }
-template <int STEPS>
 __device__ __forceinline__ float reciprocal(float x) {
   return 1.0f / x;
 }
@@ -192,7 +189,7 @@ __device__ __forceinline__ Moments<Q, C> moments(const R (&h)[Q], C Fx, C Fy, C 
   Moments<Q, C> m;
   m.drho = drho;
   m.rho = C(1) + drho;
-  const C inv = reciprocal<PAIRS ? 2 : 3>(m.rho);
+  const C inv = reciprocal(m.rho);
   m.ux = (FORCE == FORCE_NONE ? jx : jx + C(0.5) * Fx) * inv;
   if (FORCE == FORCE_ANY) {
     m.uy = (jy + C(0.5) * Fy) * inv;
@@ -204,18 +201,7 @@ __device__ __forceinline__ Moments<Q, C> moments(const R (&h)[Q], C Fx, C Fy, C 
   return m;
 }
 
-// The relaxation's factors: 1 - omega and omega times the weights of the
-// axis, the diagonal and the rest populations.
-template <int Q, typename C>
-struct Relax {
-  C omega, keep, axis, diag, rest;
-};
-template <int Q, typename C>
-__device__ __forceinline__ Relax<Q, C> relax(C omega) {
-  using L = Lat<Q>;
-  return Relax<Q, C>{omega, C(1) - omega, omega * C(L::w[0]), omega * C(L::w[Q - 2]), omega * C(L::w[Q - 1])};
-}
-// the same in scalar registers (omega is uniform over the wave)
+// a value that is uniform over the wave, in scalar registers
 __device__ __forceinline__ double scalar(double v) {
   const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
@@ -224,11 +210,6 @@ __device__ __forceinline__ double scalar(double v) {
 __device__ __forceinline__ float scalar(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(unsigned, v)));
 }
-template <int Q, typename C>
-__device__ __forceinline__ Relax<Q, C> scalar(const Relax<Q, C> &r) {
-  return Relax<Q, C>{scalar(r.omega), scalar(r.keep), scalar(r.axis), scalar(r.diag), scalar(r.rest)};
-}
-
 // Population j of the cell at index `cell` of a plane-major buffer.  With
 // W64 false the per-plane byte offset is a 32-bit unsigned value added to the
 // plane's base address, which is uniform over the wave: the load or store
@@ -247,42 +228,44 @@ __device__ __forceinline__ ST *pop_ptr(ST *base, long long plane, int j, Idx<W64
 }
 
 // Post-collision values of a cell, handed to emit(j, value) one by one.  In
-// FP64 storage the relaxation (1 - omega) h + omega w (drho - 1.5 rho u^2 + cu
-// (3 rho + 4.5 rho cu)) takes three fused multiply-adds per population (the
-// terms in rho are formed once per weight, cu once per pair); kernels that
-// take several steps per pass over memory are bound by exactly these
-// operations.  The smaller forms keep the order and the roundings of h +
-// omega (w (drho + rho (3 cu + 4.5 cu cu - 1.5 u^2)) - h), as in moments, and
-// share what is equal for both members of a pair up to the sign.
+// FP64 storage the relaxation h + omega (w (drho - 1.5 rho u^2 + cu (3 rho +
+// 4.5 rho cu)) - h) takes four fused multiply-adds per population (the terms in
+// rho are formed once, cu once per pair); kernels that take several steps per
+// pass over memory are bound by exactly these operations.  The last one adds
+// the change of h to it, so that h itself is rounded once: (1 - omega) h + ... in
+// three left twice the error (rms of u against 80-bit arithmetic, D2Q9 and
+// D3Q19, omega 0.7 to 1.8: 1.5 to 2.7 times that of the plain form, this one 0.99
+// to 1.04; a step 1 to 3 % faster).  The smaller forms keep the order and the roundings of h + omega (w
+// (drho + rho (3 cu + 4.5 cu cu - 1.5 u^2)) - h), as in moments, and share what is
+// equal for both members of a pair up to the sign.
 template <int Q, typename ST, int FORCE = FORCE_ANY, typename E>
 __device__ __forceinline__ void collide(const typename Store<ST>::R (&h)[Q], const Moments<Q, typename Store<ST>::C> &m,
-                                        const Relax<Q, typename Store<ST>::C> &rx, typename Store<ST>::C Fx,
+                                        typename Store<ST>::C omega, typename Store<ST>::C Fx,
                                         typename Store<ST>::C Fy, typename Store<ST>::C Fz, bool force, E emit) {
   using L = Lat<Q>;
   using C = typename Store<ST>::C;
-  const C omega = rx.omega;
   if (FORCE == FORCE_NONE) force = false;
   const C uF = !force ? C(0) : FORCE == FORCE_X ? m.ux * Fx : m.ux * Fx + m.uy * Fy + m.uz * Fz;
   const C fpre = C(1) - C(0.5) * omega;
   if constexpr (sizeof(ST) == 8) {
     C usq = __builtin_fma(m.uy, m.uy, m.ux * m.ux);
     if (L::D == 3 || (FORCE == FORCE_ANY && force && Fz != C(0))) usq = __builtin_fma(m.uz, m.uz, usq);
-    const C rest = __builtin_fma(C(-1.5) * m.rho, usq, m.drho), keep = rx.keep, oa = rx.axis, od = rx.diag;
-    const C a0 = oa * rest, a1 = oa * (C(3) * m.rho), a2 = oa * (C(4.5) * m.rho);
-    const C d0 = od * rest, d1 = od * (C(3) * m.rho), d2 = od * (C(4.5) * m.rho);
+    const C rest = __builtin_fma(C(-1.5) * m.rho, usq, m.drho), c1 = C(3) * m.rho, c2 = C(4.5) * m.rho;
+    auto relaxed = [&](int j, C e) {
+      const C hj = C(h[j]);
+      return __builtin_fma(omega, __builtin_fma(C(L::w[j]), e, -hj), hj);
+    };
     {
-      C out = __builtin_fma(keep, C(h[Q - 1]), rx.rest * rest);
+      C out = relaxed(Q - 1, rest);
       if (force) out -= fpre * C(L::w[Q - 1]) * C(3) * uF;
       emit(Q - 1, out);
     }
 #pragma unroll
     for (int j = 0; j < Q - 1; ++j) {
       if (!leads<Q>(j)) continue;
-      const bool diag = L::w[j] == L::w[Q - 2];
-      const C c0 = diag ? d0 : a0, c1 = diag ? d1 : a1, c2 = diag ? d2 : a2;
       const C cu = cdot<Q>(j, m.ux, m.uy, m.uz);
-      C p = __builtin_fma(cu, __builtin_fma(c2, cu, c1), __builtin_fma(keep, C(h[j]), c0));
-      C n = __builtin_fma(cu, __builtin_fma(c2, cu, -c1), __builtin_fma(keep, C(h[L::opp[j]]), c0));
+      C p = relaxed(j, __builtin_fma(cu, __builtin_fma(c2, cu, c1), rest));
+      C n = relaxed(L::opp[j], __builtin_fma(cu, __builtin_fma(c2, cu, -c1), rest));
       if (force) {
         const C fw = fpre * C(L::w[j]);
         if (FORCE == FORCE_X && !L::cx[j]) {  // across the force
@@ -344,7 +327,7 @@ __device__ __forceinline__ void collide_store(const typename Store<ST>::R (&h)[Q
                                               typename Store<ST>::C Fy, typename Store<ST>::C Fz, bool force,
                                               ST *dst, long long plane, Idx<W64> cell) {
   using C = typename Store<ST>::C;
-  collide<Q, ST>(h, m, relax<Q, C>(omega), Fx, Fy, Fz, force, [&](int j, C out) {
+  collide<Q, ST>(h, m, omega, Fx, Fy, Fz, force, [&](int j, C out) {
     ST *p = pop_ptr<ST, W64>(dst, plane, j, cell);
     if (NT) Store<ST>::st_nt(p, out);
     else Store<ST>::st(p, out);

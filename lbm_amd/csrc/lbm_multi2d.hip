@@ -234,7 +234,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
       }
     }
   }
-  const Relax<9, C> rel = scalar(relax<9, C>(C(omega_)));
+  const C omega = scalar(C(omega_));
   const C Fx = C(m.F[0]), Fy = C(m.F[1]), Fz = C(m.F[2]);
   int at = pad;  // where the state starts
   for (int s = 1; s <= T; ++s) {
@@ -273,7 +273,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
           for (int j = 0; j < 9; ++j) h[j] = Store<ST>::ld(in + j * CAP + c - sx * L::cx[j] - sy * L::cy[j]);
         }
         const Moments<9, C> mo = moments<9, C, FORCE>(h, Fx, Fy, Fz);
-        collide<9, ST, FORCE>(h, mo, rel, Fx, Fy, Fz, true, [&](int j, C value) { Store<ST>::st(&f[j], value); });
+        collide<9, ST, FORCE>(h, mo, omega, Fx, Fy, Fz, true, [&](int j, C value) { Store<ST>::st(&f[j], value); });
       }
       if (!last) {
         __syncthreads();  // every read of this round is done

@@ -188,7 +188,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(ST) == 8 ? 2 : (CLS == MULTI3D_BOX ? 4
     }
     return w;
   };
-  const Relax<19, C> rel = scalar(relax<19, C>(C(m.omega)));
+  const C omega = scalar(C(m.omega));
   const C Fx = C(m.F[0]), Fy = C(m.F[1]), Fz = C(m.F[2]);
   // the rules beyond bounce-back, on populations h of a cell with mask w in
   // plane z: the Ladd terms of moving walls and the NEEM correction
@@ -293,7 +293,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(ST) == 8 ? 2 : (CLS == MULTI3D_BOX ? 4
       if (WALLS && __ballot(wp != 0)) rules(wp, wrapped(p, nz), h);
       const Moments<19, C> mo = moments<19, C, FORCE>(h, Fx, Fy, Fz);
       if (std::is_same<C, double>::value) reconvert(h);
-      collide<19, ST, FORCE>(h, mo, rel, Fx, Fy, Fz, true, [&](int j, C value) { Store<ST>::st(&v[j], value); });
+      collide<19, ST, FORCE>(h, mo, omega, Fx, Fy, Fz, true, [&](int j, C value) { Store<ST>::st(&v[j], value); });
     }
     lds_barrier();  // the previous plane's reads of the slot are done
     if (first && mine) {
@@ -331,7 +331,7 @@ __attribute__((amdgpu_waves_per_eu(sizeof(ST) == 8 ? 2 : (CLS == MULTI3D_BOX ? 4
       __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
       if (inner && !(WALLS && (vq & LINK_SELF_SOLID))) {
         const long long zo = (long long)wrapped(q, nz) * zs;
-        collide<19, ST, FORCE>(h, mo, rel, Fx, Fy, Fz, true, [&](int j, C value) {
+        collide<19, ST, FORCE>(h, mo, omega, Fx, Fy, Fz, true, [&](int j, C value) {
           const ST *base = dst + (long long)j * m.plane + zo;  // uniform
           ST out;
           Store<ST>::st(&out, value);
