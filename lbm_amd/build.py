@@ -13,7 +13,7 @@ ROOT = os.path.dirname(HERE)
 HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 # packed FP32 instructions are disabled for every HIP translation unit; host
 # functions start on 64 bytes (the random generator of the network's first
-# weights took 108 ms instead of 62 where the linker had put it elsewhere)
+# weights took 1.7 times as long where the linker had put it elsewhere)
 HIPFLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
             "-packed-fp32-ops", "-ffp-contract=off", "-Xarch_host", "-falign-functions=64", "-Wno-unused-result",
             "-Wno-unused-value"]

@@ -6,7 +6,9 @@
 // launch (3.5-4.5 us a step whatever the cell count), on large ones HBM (72 B
 // per FP32 cell update, every step).  Here both are paid once per `steps`
 // updates; what is left is the FP64 (FP32 for 16-bit storage) arithmetic of
-// the updates, 1.1-1.3 times as many as cells for the halo.
+// the updates, for the halo too: 1.2 times as many as cells in 64 x 20 tiles and
+// 4 steps, 1.35 in 32 x 32 and 6, 1.8 in 32 x 16 and 8, 3.8 in 8 x 8 and 8, where
+// the launch is what counts.
 //
 // In place: a step overwrites the tile's old state, so LDS holds it once.
 // The cells of a step are taken in the order of their slots (row-major, or by
@@ -382,7 +384,7 @@ static Multi2dPlan general_plan(const Multi2dDomain &d) {
 
 // Domains of few rows: a tile of the rule above holds too few cells for its
 // threads there, and the rows of a periodic axis are updated several times
-// over (3 rows and 6 steps: 3 times).  Wider tiles with fewer steps, or one
+// over (3 rows and 6 steps: 3 times).  Wider or lower tiles with fewer steps, or one
 // step per launch where even these take longer, by multi2d_time (below 2^15
 // cells the launch is all there is to save, and the rule above holds).
 // Microseconds per step, one step per launch, the rule above, this one:
@@ -391,10 +393,11 @@ static Multi2dPlan general_plan(const Multi2dDomain &d) {
 //   1333333 x 3 FP16 walls     46     63     33   (256 x 3, 4 steps)
 //   250000 x 4 FP32 NEEM       16.7   29.6   14.1 (128 x 4, 4 steps)
 //   100000 x 10 FP32 periodic  15.5   13.8   12.0
-// From 32 rows on the rule above is never slower than 1.05 times one step per
-// launch (25000 x 40 FP16, periodic with a force along y: 9.8 against 9.3).
+//   20000 x 50 FP16 periodic, force along x and y   9.0   11.7   8.9
+// From 64 rows on the rule above is at most 1.02 times as slow as one step per
+// launch; below, of 3000 timed cases this one is in 15, by 1.03 to 1.11.
 Multi2dPlan multi2d_plan(const Multi2dDomain &d) {
-  constexpr int THIN = 32;
+  constexpr int THIN = 64;
   const Multi2dPlan general = general_plan(d);
   if (d.ny >= THIN || d.cells < 1 << 15) return general;
   Multi2dPlan best = general;

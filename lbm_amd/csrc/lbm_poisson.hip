@@ -244,7 +244,8 @@ __global__ void __launch_bounds__(256) k_poisson_step(const PArgs a) {
 // was bound by the launch on small windows and by HBM on large ones, both
 // paid once per `steps` here; the arithmetic (20 FP64 operations a cell) is
 // far below either.  What bounds it now: large windows, LDS (8 reads and 8
-// writes of 8 bytes per cell and step, 2.6 times over with the halo).
+// writes of 8 bytes per cell update, 1.6 updates per cell and step with the
+// halo of 16 x 24 tiles, which load 2.6 times their cells).
 // LDS holds one state: a step's cells, at most two per thread, stay in
 // registers until every thread has read (no order of the cells to keep,
 // which the rules of a face, reaching three cells inward, would ask for).

@@ -209,7 +209,7 @@ for ny in list(range(3, 34)) + [48, 63]:
         lat.step(24)
         lat.close()
         plans = multi2d(since)
-        assert plans or (ny < 32 and cells >= 30000), (nx, ny)
+        assert plans or (ny < 64 and cells >= 30000), (nx, ny)
         if not plans:
             assert len(launches("k_step", since)) == 24
             continue
@@ -222,10 +222,11 @@ for ny in list(range(3, 34)) + [48, 63]:
                 n = slots(x0, min(x0 + a.tw, nx) - 1, y0, min(y0 + a.th, ny) - 1, nx, ny, a.steps, "{faces}" != "neem", box,
                           "{faces}" == "neem")
                 assert n <= cap, (nx, ny, a.tw, a.th, a.steps, x0, y0, n)
-lat = capi.Lattice((1 << 20, 3), storage="f16", omega=1.2)
-since = count()
-lat.step(24)
-assert len(launches("k_step", since)) == 24
+for shape, force in (((1 << 20, 3), (0.0, 0.0, 0.0)), ((20000, 50), (1e-6, 1e-6, 0.0))):
+    lat = capi.Lattice(shape, storage="f16", omega=1.2, force=force)
+    since = count()
+    lat.step(24)
+    assert len(launches("k_step", since)) == 24, shape
 """)
 
 

@@ -46,7 +46,7 @@ def test_low_domains_equal_single_steps(storage, faces):
     walls = {"-y": WALL, "+y": ("wall", (0.02, 0.0), 1.0)}
     kinds = {"periodic": {}, "walls": walls,
              "neem": dict(walls, **{"-x": ("velocity_neem", (0.03, 0.0), 1.0), "+x": ("pressure_neem", None, 1.0)})}
-    for nx, ny in ((701, 3), (40000, 3), (300000, 3), (30011, 5), (250007, 6), (33, 12), (20001, 17), (60000, 31)):
+    for nx, ny in ((701, 3), (40000, 3), (300000, 3), (30011, 5), (250007, 6), (33, 12), (20001, 17), (60000, 31), (30003, 45), (9001, 62)):
         solid = (np.random.default_rng(ny).random(nx * ny) < 0.05).astype(np.uint8) if ny > 5 else None
         out = []
         for calls in ((17, 2, 5), (1,) * 24):
