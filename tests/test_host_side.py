@@ -215,7 +215,8 @@ for ny in list(range(3, 34)) + [48, 63]:
             continue
         a = plans[0]
         if cells >= 400000 and ny < 32:
-            assert updates(a, box) < 2.0, (nx, ny, a.tw, a.th, a.steps)
+            # (FP64: the step that it replaces moves twice the bytes)
+            assert updates(a, box) < (3.0 if {esize} == 8 else 2.0), (nx, ny, a.tw, a.th, a.steps)
         edge = lambda n, w: sorted({{0, w, n // w // 2 * w, (n - 1) // w * w - w, (n - 1) // w * w}} & set(range(0, n, w)))
         for x0 in edge(nx, a.tw):
             for y0 in edge(ny, a.th):
