@@ -111,3 +111,29 @@ def test_d3q19_fp32_walls_and_solids(shape):
     solid = scattered(shape, 9)
     a, b = both(shape, "f32", {"-z": WALL, "+z": ("wall", (0.02, 0.01, 0.0), 1.0)}, (2, 3), solid)
     assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
+LID3 = {"-x": WALL, "+x": ("wall", (0.0, 0.0, 0.02), 1.0), **Z_WALLS}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage,shape,faces,force", [
+    ("f32", (5, 5, 31500), {}, (0.0, 0.0, 0.0)), ("f32", (33, 31, 770), {}, (1e-5, 0.0, 0.0)),
+    ("f32", (100, 98, 81), {}, (0.0, 0.0, 0.0)), ("f32", (4, 1020, 200), {}, (1e-5, 2e-6, 0.0)),
+    ("f32", (4, 1020, 200), Z_WALLS, (1e-5, 0.0, 0.0)), ("f32", (5, 5, 31500), LID3, (0.0, 0.0, 0.0)),
+    ("f32", (150, 143, 149), LID3, (0.0, 0.0, 0.0)), ("f32", (8800, 30, 3), {**Y_WALLS, "-z": WALL, "+z": WALL}, (0.0, 0.0, 0.0)),
+    ("f16", (150, 143, 149), {}, (1e-5, 0.0, 0.0)), ("bf16", (3, 1300, 810), {}, (0.0, 0.0, 0.0))])
+def test_d3q19_smaller_storage_forms(storage, shape, faces, force):
+    from lbm_amd import capi
+
+    n, rng, out = int(np.prod(shape)), np.random.default_rng(4), []
+    rho, u = 1 + 1e-3 * rng.standard_normal(n), 0.01 + 2e-3 * rng.standard_normal((n, 3))
+    for calls in ((4, 3), (1,) * 7):
+        lat = capi.Lattice(shape, storage=storage, omega=1.1, faces=faces, force=force)
+        assert lat.steps_per_launch(2) == 2
+        lat.init(rho, u)
+        for k in calls:
+            lat.step(k)
+        out.append(lat.populations())
+        lat.close()
+    assert np.isfinite(out[0]).all() and np.array_equal(*out)
